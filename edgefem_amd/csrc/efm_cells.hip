@@ -28,9 +28,14 @@ using namespace efm;
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kRowsPerTile = 1024;
+constexpr int kRowsPerTile = 1024;  // at most
 constexpr int kLanes = 8;  // SpMV lanes per row
 constexpr int kMaxR = 2;
+constexpr int kMinTiles = 1600;  // row tiles wanted of a batch that can have them (subs_per_tile)
+// Nodes per block of the nodal kernel: two rounds of 32 nodes.  A tile of 1,024 nodes is 32
+// serial rounds of dependent loads on a grid of one block per 1,024 nodes: 54.0 us per
+// launch on 12 cells (60 blocks) against 6.7 us with 64 nodes.
+constexpr int kNodesPerTile = 64;
 
 struct CellSys {
   double2 rho, alpha, beta, omega;
@@ -906,19 +911,58 @@ template <typename T> int upload(efm::DevBuf &d, const T *h, size_t count, hipSt
   return EFM_OK;
 }
 
-std::vector<Tile> make_tiles(const int64_t *off, int64_t ncells, std::vector<int32_t> *first) {
+// Tiles of at most `per_tile` rows (or nodes), none across two cells.
+std::vector<Tile> make_tiles(const int64_t *off, int64_t ncells, int64_t per_tile, std::vector<int32_t> *first) {
   std::vector<Tile> t;
   if (first)
     first->assign(ncells + 1, 0);
   for (int64_t c = 0; c < ncells; ++c) {
     if (first)
       (*first)[c] = (int32_t)t.size();
-    for (int64_t r = off[c]; r < off[c + 1]; r += kRowsPerTile)
-      t.push_back(Tile{(int32_t)c, 0, r, std::min<int64_t>(off[c + 1], r + kRowsPerTile)});
+    for (int64_t r = off[c]; r < off[c + 1]; r += per_tile)
+      t.push_back(Tile{(int32_t)c, 0, r, std::min<int64_t>(off[c + 1], r + per_tile)});
   }
   if (first)
     (*first)[ncells] = (int32_t)t.size();
   return t;
+}
+
+// Sub-tiles per row tile (one block each in every row kernel).  A tile is one block's
+// serial walk, so few tiles leave most CUs idle and the last round of blocks nearly empty;
+// many tiles cost the finalisation more slots and lose the overlap of one sub-tile's loads
+// with the previous one's gathers.  Measured on 12 cells, 0.4 M rows (whole batch): 16
+// sub-tiles 317 ms, 7 (one round of resident blocks) 275, 4: 211, 2: 217, 1: 200 (4 and
+// below are alike up to the iteration counts); 512 cells, 27 M rows, run with 16.
+int subs_per_tile(int64_t n) {
+  const int64_t subs = n / kSubRows;
+  return (int)std::max<int64_t>(1, std::min<int64_t>(kRowsPerTile / kSubRows, subs / kMinTiles));
+}
+
+// Row tiles of up to `subs` whole entry sub-tiles (sub-tile: at most kSubNnz entries and
+// kSubRows rows of one cell).  False when a row holds more than kSubNnz entries.
+bool make_row_tiles(const int64_t *off, int64_t ncells, const int32_t *rp, int subs, std::vector<Tile> &tiles,
+                    std::vector<int32_t> &first, std::vector<int4> &sd, std::vector<int32_t> &so) {
+  first.assign(ncells + 1, 0);
+  for (int64_t c = 0; c < ncells; ++c) {
+    first[c] = (int32_t)tiles.size();
+    for (int64_t r = off[c]; r < off[c + 1];) {
+      const int64_t r0 = r;
+      so.push_back((int32_t)sd.size());
+      for (int k = 0; k < subs && r < off[c + 1]; ++k) {
+        int64_t r1 = r;
+        while (r1 < off[c + 1] && r1 - r < kSubRows && rp[r1 + 1] - rp[r] <= kSubNnz)
+          ++r1;
+        if (r1 == r)
+          return false;
+        sd.push_back(make_int4((int32_t)r, (int32_t)r1, rp[r], rp[r1]));
+        r = r1;
+      }
+      tiles.push_back(Tile{(int32_t)c, 0, r0, r});
+    }
+  }
+  first[ncells] = (int32_t)tiles.size();
+  so.push_back((int32_t)sd.size());
+  return true;
 }
 } // namespace
 
@@ -962,11 +1006,6 @@ extern "C" int efm_cells_create(int64_t ncells, const int64_t *h_row_off, const 
     EFM_REQUIRE(std::adjacent_find(rows.begin(), rows.end()) == rows.end(),
                 "efm_cells_create: port terms must be disjoint");
   }
-  std::vector<int32_t> first;
-  std::vector<Tile> tiles = make_tiles(h_row_off, ncells, &first);
-  std::vector<Tile> ntl = make_tiles(h_node_off, ncells, nullptr);
-  s->ntiles = (int64_t)tiles.size();
-  s->nntiles = (int64_t)ntl.size();
   int rc;
   const size_t vb = (size_t)n * s->R * sizeof(double2);
   if ((rc = s->row_ptr.alloc((n + 1) * sizeof(int32_t))) || (rc = s->col.alloc(std::max<int64_t>(nnz, 1) * 4)) ||
@@ -981,36 +1020,28 @@ extern "C" int efm_cells_create(int64_t ncells, const int64_t *h_row_off, const 
     EFM_HIP_CHECK(hipStreamSynchronize(st));
     EFM_REQUIRE(last == nnz, "efm_cells_create: row_ptr[n] != nnz");
   }
-  {  // entry sub-tiles of every row tile for the SpMV: <= kSubNnz entries, <= kSubRows rows
+  // row tiles, and the entry sub-tiles of each for the SpMV
+  std::vector<int32_t> first, so;
+  std::vector<Tile> tiles;
+  std::vector<int4> sd;
+  {
     std::vector<int32_t> hrp(n + 1);
     EFM_HIP_CHECK(hipMemcpy(hrp.data(), s->row_ptr.p, (n + 1) * sizeof(int32_t), hipMemcpyDeviceToHost));
-    std::vector<int4> sd;
-    std::vector<int32_t> so(tiles.size() + 1, 0);
-    bool ok = true;
-    for (size_t ti = 0; ti < tiles.size() && ok; ++ti) {
-      so[ti] = (int32_t)sd.size();
-      for (int64_t r = tiles[ti].r0; r < tiles[ti].r1;) {
-        int64_t r1 = r;
-        while (r1 < tiles[ti].r1 && r1 - r < kSubRows && hrp[r1 + 1] - hrp[r] <= kSubNnz)
-          ++r1;
-        if (r1 == r) {  // a row longer than a sub-tile: keep the row-parallel kernel
-          ok = false;
-          break;
-        }
-        sd.push_back(make_int4((int32_t)r, (int32_t)r1, hrp[r], hrp[r1]));
-        r = r1;
-      }
+    if (!make_row_tiles(h_row_off, ncells, hrp.data(), subs_per_tile(n), tiles, first, sd, so)) {
+      // a row longer than a sub-tile: keep the row-parallel kernel
+      tiles = make_tiles(h_row_off, ncells, kRowsPerTile, &first);
+      sd.clear();
     }
-    so[tiles.size()] = (int32_t)sd.size();
-    s->nsub = 0;
-    if (ok && !sd.empty()) {
+    if (!sd.empty()) {
       if ((rc = upload(s->sdesc, sd.data(), sd.size(), st)) || (rc = upload(s->soff, so.data(), so.size(), st)))
         return rc;
-      EFM_HIP_CHECK(hipStreamSynchronize(st));  // sd and so are freed at the end of this block
       s->nsub = (int64_t)sd.size();
       s->spmv = 1;
     }
   }
+  std::vector<Tile> ntl = make_tiles(h_node_off, ncells, kNodesPerTile, nullptr);
+  s->ntiles = (int64_t)tiles.size();
+  s->nntiles = (int64_t)ntl.size();
   // gradient incidence (global node indices) and its transpose, on the device
   {
     DevBuf ab, cnt, cursor, work, err;
