@@ -192,9 +192,14 @@ int efm_solver_solve(efm_solver *s, const double *B, double *X, const efm_solve_
  * length inside windows of 4096, no LDS; built on the device at first use); 11: variant 9
  * with the values stored as a real part per entry plus the imaginary parts of the tiles
  * that have any (a tile of real values streams 8 B per value instead of 16; complex-double
- * matrices; rebuilt on the device after every set_matrix).  By
- * default (-1) the first solve times every variant on the installed matrix and keeps the
- * fastest; a fixed variant makes results reproducible bit for bit across runs.
+ * matrices; rebuilt on the device after every set_matrix); 12: all iterations in one
+ * persistent kernel that keeps the matrix in registers and LDS, COCG on complex-double
+ * matrices of up to 512 rows per CU (256 with three or four right-hand sides) whose blocks of
+ * rows read few enough columns, with at most four low-rank terms times right-hand sides;
+ * a solve that it does not cover is refused).  By default (-1) systems that variant 12
+ * covers are solved with it (get reports -1); for others the first solve times variants
+ * 0-11 on the installed matrix and keeps the fastest; a fixed variant makes results
+ * reproducible bit for bit across runs.
  * h_tune_ms (12 entries, may be NULL) receives the
  * measured average ms per launch (-1 = not available).  No reference counterpart. */
 int efm_solver_set_spmv_variant(efm_solver *s, int variant);
