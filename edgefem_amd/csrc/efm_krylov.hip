@@ -1755,7 +1755,6 @@ constexpr int kZForm = 9;             // COCG with p formed in its own pass (its
 constexpr int kSellForm = 10;         // the same iteration with the sliced-ELL SpMV
 constexpr int kSplitForm = 11;        // the same iteration, values stored as real parts plus the imaginary parts of complex tiles
 constexpr int kSellRL = 4;            // lanes per row of the sliced-ELL SpMV
-constexpr int kPersistForm = 12;      // the whole COCG in one persistent kernel (efm_persist.h)
 constexpr int kPersistLaunch = 4096;  // iterations per launch at most
 
 struct efm_solver {
@@ -1807,7 +1806,7 @@ struct efm_solver {
   int lr_P = 0;
   int64_t lr_len = 0;
   efm::DevBuf lr_idx, lr_val, lr_coef;
-  // variant 12 (persistent kernel), set up on first use: row blocks and their local columns
+  // persistent kernel (efm_persist.h), set up on first use: row blocks and their local columns
   int ncu = 256;
   int ps_state = 0;  // 0: not tried, 1: set up, -1: the matrix does not fit
   int ps_nb = 0, ps_rpb = 0, ps_nsm = 0, ps_lds = 0;
@@ -2837,12 +2836,7 @@ extern "C" int efm_solver_spmv(efm_solver *s, const double *x, double *y, void *
 
 extern "C" int efm_solver_set_spmv_variant(efm_solver *s, int variant) {
   EFM_REQUIRE(s, "efm_solver_set_spmv_variant: NULL solver");
-  EFM_REQUIRE(variant >= -1 && (variant < kNumSpmvVariants || variant == kPersistForm),
-              "efm_solver_set_spmv_variant: bad variant");
-  if (variant == kPersistForm) {
-    s->spmv_variant = variant;
-    return EFM_OK;
-  }
+  EFM_REQUIRE(variant >= -1 && variant < kNumSpmvVariants, "efm_solver_set_spmv_variant: bad variant");
   EFM_REQUIRE(variant < 0 || !kRetired(variant),
               "efm_solver_set_spmv_variant: variants 5, 7 and 8 were removed (slower on every matrix measured)");
   EFM_REQUIRE(variant < 3 || variant == kSellForm ||
@@ -2921,7 +2915,7 @@ extern "C" int efm_solver_solve(efm_solver *s, const double *B, double *X,
   // Systems whose matrix fits in the register files run in the persistent kernel: 780 rows 21.6
   // (five launches) against 13.3 us per iteration, 31 k 29 against 18.4, 103 k 43 against 33.0.
   bool persist = false;
-  if (cocg && !s->profile && (s->spmv_variant == kPersistForm || s->spmv_variant < 0)) {
+  if (cocg && !s->profile && s->spmv_variant < 0) {
     rc = with_rhs(s->R, [&](auto RC) -> int {
       constexpr int R = decltype(RC)::value;
       if (!Dispatch<R>::persist_covers(s))
@@ -2933,8 +2927,6 @@ extern "C" int efm_solver_solve(efm_solver *s, const double *B, double *X,
     if (rc != EFM_OK)
       return rc;
   }
-  EFM_REQUIRE(persist || s->spmv_variant != kPersistForm,
-              "efm_solver_solve: the persistent form (12) does not fit this system");
   if (persist) {
     bool done = false;
     rc = with_rhs(s->R, [&](auto RC) -> int {
@@ -2944,7 +2936,6 @@ extern "C" int efm_solver_solve(efm_solver *s, const double *B, double *X,
     if (rc != EFM_OK)
       return rc;
     if (!done) {  // from the start again, one launch per step
-      EFM_REQUIRE(s->spmv_variant < 0, "efm_solver_solve: the persistent kernel was not run to its end");
       persist = false;
       if ((rc = start()) != EFM_OK)
         return rc;

@@ -1643,6 +1643,309 @@ __global__ void __launch_bounds__(kBlock)
   active_flag[s] = S.active | (S.want << 1);
 }
 
+// ---------------------------------------------------------------------------
+// Narrow batches.  The kernels above give a system a lane and a row a wavefront: a batch of
+// 8 systems takes as long as one of 64 (31 k rows: 61 ms for 9 frequencies with two
+// excitations, 68 ms for 32).  Here a block's threads are RB rows of B systems (thread =
+// sub * B + s), vectors are [row][nsys] without padding, and the
+// block stages the column indices and values of its RB rows in LDS, from where every system
+// of a row reads them (an entry is then two LDS reads at one address per row and one
+// gather of B consecutive systems).  XCD-aware walks over chunks of RB rows as above.
+// Standard COCG, form 2, complex-FP64 vectors.  41 k rows, 18 systems, us per launch, one row
+// per wavefront against this: SpMV 40, 25; p 26, 13; update 23, 11; nodes 20, 10.  With few
+// systems a kernel is a chain of three or four memory round trips (8 systems: 11, 6, 7, 9).
+// Measured no better: four or eight gathers at a time instead of five, the next chunk's
+// entries loaded ahead (28 against 25 us), two or eight blocks per CU instead of four.
+// ---------------------------------------------------------------------------
+constexpr int kFlatVariant = 3;     // as SpMV and nodal variant inside a solve
+constexpr int kFlatThreads = 512;   // threads of a block at most
+constexpr int kFlatRows = 64;       // rows of a chunk at most
+constexpr int kFlatStage = 24;      // staged entries per row (a chunk with more reads them from memory)
+
+// Geometry of a batch of B <= 256 systems: RB rows per block of T threads, T the width with the
+// fewest idle threads; `stage` entries fit in LDS.
+struct FlatDims {
+  int RB, T, stage;
+};
+FlatDims flat_dims(int B) {
+  FlatDims d{};
+  double best = -1.0;
+  for (int t = 256; t <= kFlatThreads; t += 64) {
+    const int rb = std::min(t / B, kFlatRows);
+    const int tt = (rb * B + 63) / 64 * 64;
+    const double eff = (double)(rb * B) / tt;
+    if (eff > best + 0.02) {
+      best = eff;
+      d.RB = rb;
+      d.T = tt;
+    }
+  }
+  d.stage = d.RB * kFlatStage;
+  return d;
+}
+
+// The packed kernels where the others would leave more than 3/8 of the lanes of one wavefront
+// or 1/4 of two or three idle (31 k rows, others against packed, ms: 6 systems 70, 30; 18: 61,
+// 41; 34: 63, 54; 40: 63, 61; 48: 65, 68; 66: 114, 83; 88: 111, 96; 96: 114, 110; 128: 123, 138;
+// 144: 176, 156; 4.8 k rows: 10 systems 17, 14; 40 and 80 17, 17 and 25, 24; 45 k rows: 40 and 96
+// systems 93, 92 and 181, 182), so for at most 143 systems; offsets in bytes in 32 bits.
+bool flat_wins(int64_t n, int nsys) {
+  const int padded = (nsys + kSys - 1) / kSys * kSys;
+  return 8 * nsys < (padded > kSys ? 6 : 5) * padded && nsys <= 143 && n * nsys < ((int64_t)1 << 28);
+}
+
+// Chunks of RB rows, contiguous per XCD (block bx runs on XCD bx % 8).
+struct FlatWalk {
+  int64_t begin, end, stride;
+  __device__ FlatWalk(int64_t items, int RB) {
+    const int64_t span = ((items + RB - 1) / RB + 7) / 8;
+    const int xcd = blockIdx.x & 7;
+    begin = xcd * span + (blockIdx.x >> 3);
+    end = min((items + RB - 1) / RB, (int64_t)(xcd + 1) * span);
+    stride = gridDim.x >> 3;
+  }
+};
+
+// Per-block partial sums of V values per system, in the layout of write_sys_partials.
+template <int V>
+__device__ inline void flat_partials(const double2 (&v)[V], double2 *red, double2 *partial, int B, int RB,
+                                     int sub, int s) {
+#pragma unroll
+  for (int k = 0; k < V; ++k) {
+    __syncthreads();
+    red[threadIdx.x] = v[k];
+    __syncthreads();
+    if (sub == 0) {
+      double2 a = red[s];
+      for (int q = 1; q < RB; ++q)
+        a = cadd(a, red[q * B + s]);
+      partial[(((int64_t)(s / kSys) * gridDim.x + blockIdx.x) * V + k) * 64 + s % kSys] = a;
+    }
+  }
+}
+
+// The map of k_sw_pform_u with the pending x update.
+__global__ void __launch_bounds__(kFlatThreads)
+    k_sf_pform(int64_t n, int B, int RB, int P, const int2 *__restrict__ en_eff,
+               const double2 *__restrict__ dK, const double2 *__restrict__ dM, const double *__restrict__ dMs,
+               const int8_t *__restrict__ rport, const double *__restrict__ k0sq,
+               const double2 *__restrict__ coef, const double2 *__restrict__ y, const double2 *__restrict__ r,
+               double2 *__restrict__ p, double2 *__restrict__ x, const SwState *__restrict__ st) {
+  const int sub = threadIdx.x / B, s = threadIdx.x % B;
+  if (sub >= RB || st[s].active == 0)
+    return;
+  const double2 alpha = st[s].alpha, beta = st[s].beta;
+  const double k2 = k0sq[s];
+  const bool xu = st[s].iters > 0;
+  FlatWalk cw(n, RB);
+  for (int64_t c = cw.begin; c < cw.end; c += cw.stride) {
+    const int64_t e = c * RB + sub;
+    if (e >= n)
+      break;
+    const int64_t i = e * B + s;
+    const int2 ab = en_eff[e];
+    double2 z = bil(edge_diag_inv(e, s, P, k2, dK, dM, dMs, rport, coef), r[i]);
+    const bool hn = ab.x >= 0;
+    const double2 yd = csub(y[(int64_t)(hn ? ab.y : 0) * B + s], y[(int64_t)(hn ? ab.x : 0) * B + s]);
+    z = hn ? cadd(z, yd) : z;
+    const double2 po = p[i];
+    if (xu)
+      x[i] = cfma(alpha, po, x[i]);
+    p[i] = cfma(beta, po, z);
+  }
+}
+
+// Real parts (and imaginary parts, where there are any) of an entry of K and M side by side.
+__global__ void k_sf_pair(int64_t nnz, const double2 *__restrict__ K, const double2 *__restrict__ M,
+                          double2 *__restrict__ KM, double2 *__restrict__ KMi) {
+  const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= nnz)
+    return;
+  const double2 a = K[k], b = M[k];
+  KM[k] = make_double2(a.x, b.x);
+  if (KMi)
+    KMi[k] = make_double2(a.y, b.y);
+}
+
+// w = A_s u; partials of u^T w.  CPLX: K or M has nonzero imaginary parts.
+template <bool CPLX>
+__global__ void __launch_bounds__(kFlatThreads)
+    k_sf_spmv(int64_t n, int B, int RB, int stage, int P, const int32_t *__restrict__ row_ptr,
+              const int32_t *__restrict__ col, const double2 *__restrict__ KM, const double2 *__restrict__ KMi,
+              const double *__restrict__ Ms, const int8_t *__restrict__ rport, const double *__restrict__ k0sq,
+              const double2 *__restrict__ coef, const double2 *__restrict__ u, double2 *__restrict__ w,
+              double2 *__restrict__ partial, const SwState *__restrict__ st) {
+  constexpr int U = 5;
+  extern __shared__ double2 flat_lds[];  // values (and imaginary parts), columns; at the end the partials
+  double2 *lkm = flat_lds, *lim = flat_lds + stage + 1;
+  unsigned *lcol = reinterpret_cast<unsigned *>(flat_lds + (CPLX ? 2 : 1) * (stage + 1));  // byte offsets in u
+  const int sub = threadIdx.x / B, s = threadIdx.x % B;
+  const bool act = sub < RB && st[s].active != 0;
+  const double k2 = act ? k0sq[s] : 0.0;
+  double2 v[1] = {make_double2(0, 0)};
+  FlatWalk cw(n, RB);
+  const char *ub = reinterpret_cast<const char *>(u);
+  for (int64_t c = cw.begin; c < cw.end; c += cw.stride) {
+    const int64_t row0 = c * RB, row = row0 + sub;
+    const int32_t k0 = row_ptr[row0], m = row_ptr[min(n, row0 + RB)] - k0;
+    const bool staged = m <= stage;
+    __syncthreads();  // the previous chunk has been read
+    if (staged) {
+      for (int i = threadIdx.x; i < m; i += blockDim.x) {
+        lkm[i] = KM[k0 + i];
+        if (CPLX)
+          lim[i] = KMi[k0 + i];
+        lcol[i] = (unsigned)col[k0 + i] * (unsigned)B * 16u;
+      }
+      if (threadIdx.x == 0) {  // what slots past a row's end read
+        lkm[stage] = make_double2(0, 0);
+        if (CPLX)
+          lim[stage] = make_double2(0, 0);
+        lcol[stage] = (unsigned)row0 * (unsigned)B * 16u;
+      }
+    }
+    const bool on = act && row < n;
+    const int a = on ? row_ptr[row] - k0 : 0, b = on ? row_ptr[row + 1] - k0 : 0;
+    const int port = on ? rport[row] : -1;
+    const double2 ud = on ? u[row * B + s] : make_double2(0, 0);
+    __syncthreads();
+    double2 acc = make_double2(0, 0);
+    if (staged) {
+      for (int j = a; j < b; j += U) {
+        double2 xv[U];
+        int q[U];
+#pragma unroll
+        for (int t = 0; t < U; ++t) {
+          q[t] = j + t < b ? j + t : stage;
+          xv[t] = *reinterpret_cast<const double2 *>(ub + (lcol[q[t]] + 16u * (unsigned)s));
+        }
+#pragma unroll
+        for (int t = 0; t < U; ++t) {
+          const double2 km = lkm[q[t]];
+          const double ax = km.x - k2 * km.y;
+          if (CPLX) {
+            const double2 im = lim[q[t]];
+            acc = cfma(make_double2(ax, im.x - k2 * im.y), xv[t], acc);
+          } else {
+            acc.x += ax * xv[t].x;
+            acc.y += ax * xv[t].y;
+          }
+        }
+      }
+    } else {
+      for (int j = a; j < b; ++j) {
+        const double2 km = KM[k0 + j], im = CPLX ? KMi[k0 + j] : make_double2(0, 0);
+        acc = cfma(make_double2(km.x - k2 * km.y, im.x - k2 * im.y), u[(int64_t)col[k0 + j] * B + s], acc);
+      }
+    }
+    if (port >= 0) {
+      const double2 cp = coef[s * P + port];
+      double2 as = make_double2(0, 0);
+      for (int j = a; j < b; ++j) {
+        const double mw = Ms[k0 + j];
+        const double2 xv = u[(int64_t)col[k0 + j] * B + s];
+        as.x += mw * xv.x;
+        as.y += mw * xv.y;
+      }
+      acc = cfma(cp, as, acc);
+    }
+    if (on) {
+      w[row * B + s] = acc;
+      v[0] = cadd(v[0], bil(ud, acc));
+    }
+  }
+  flat_partials<1>(v, flat_lds, partial, B, RB, sub, s);
+}
+
+// y = Dn^{-1} G^T (r - alpha w); WITH_W false: y = Dn^{-1} G^T r.
+template <bool WITH_W>
+__global__ void __launch_bounds__(kFlatThreads)
+    k_sf_node(int64_t N, int B, int RB, int stage, const int32_t *__restrict__ n2e_ptr,
+              const int32_t *__restrict__ n2e, const int8_t *__restrict__ gsign,
+              const double2 *__restrict__ dninv, const double2 *__restrict__ r, const double2 *__restrict__ w,
+              double2 *__restrict__ y, const SwState *__restrict__ st) {
+  constexpr int U = 6;
+  extern __shared__ int flat_node_lds[];
+  int *le = flat_node_lds, *lg = flat_node_lds + stage;
+  const int sub = threadIdx.x / B, s = threadIdx.x % B;
+  const bool act = sub < RB && st[s].active != 0;
+  const double2 alpha = WITH_W && act ? st[s].alpha : make_double2(0, 0);
+  FlatWalk cw(N, RB);
+  for (int64_t c = cw.begin; c < cw.end; c += cw.stride) {
+    const int64_t n0 = c * RB, nd = n0 + sub;
+    const int32_t k0 = n2e_ptr[n0], m = n2e_ptr[min(N, n0 + RB)] - k0;
+    const bool staged = m <= stage;
+    __syncthreads();  // the previous chunk has been read
+    if (staged)
+      for (int i = threadIdx.x; i < m; i += blockDim.x) {
+        le[i] = n2e[k0 + i];
+        lg[i] = gsign[k0 + i];
+      }
+    const bool on = act && nd < N;
+    const int a = on ? n2e_ptr[nd] - k0 : 0, b = on ? n2e_ptr[nd + 1] - k0 : 0;
+    const double2 di = on ? dninv[nd * B + s] : make_double2(0, 0);
+    __syncthreads();
+    double2 sr = make_double2(0, 0), sw = make_double2(0, 0);
+    for (int j = a; j < b; j += U) {
+      double2 xr[U], xw[U];
+      double g[U];
+#pragma unroll
+      for (int t = 0; t < U; ++t) {
+        const int q = min(j + t, b - 1);
+        const int64_t i = (int64_t)(staged ? le[q] : n2e[k0 + q]) * B + s;
+        g[t] = j + t < b ? (double)(staged ? lg[q] : (int)gsign[k0 + q]) : 0.0;
+        xr[t] = r[i];
+        if (WITH_W)
+          xw[t] = w[i];
+      }
+#pragma unroll
+      for (int t = 0; t < U; ++t) {
+        sr.x += g[t] * xr[t].x;
+        sr.y += g[t] * xr[t].y;
+        if (WITH_W) {
+          sw.x += g[t] * xw[t].x;
+          sw.y += g[t] * xw[t].y;
+        }
+      }
+    }
+    if (on)
+      y[nd * B + s] = cmul(di, WITH_W ? csub(sr, cmul(alpha, sw)) : sr);
+  }
+}
+
+// The map of k_sw_update_std without the x update: r -= alpha w, partials of u^T r and |r|^2.
+__global__ void __launch_bounds__(kFlatThreads)
+    k_sf_update(int64_t n, int B, int RB, int P, const int2 *__restrict__ en_eff,
+                const double2 *__restrict__ dK, const double2 *__restrict__ dM, const double *__restrict__ dMs,
+                const int8_t *__restrict__ rport, const double *__restrict__ k0sq,
+                const double2 *__restrict__ coef, const double2 *__restrict__ y, const double2 *__restrict__ w,
+                double2 *__restrict__ r, double2 *__restrict__ partial, const SwState *__restrict__ st) {
+  __shared__ double2 red[kFlatThreads];
+  const int sub = threadIdx.x / B, s = threadIdx.x % B;
+  double2 v[2] = {make_double2(0, 0), make_double2(0, 0)};
+  if (sub < RB && st[s].active != 0) {
+    const double2 alpha = st[s].alpha;
+    const double k2 = k0sq[s];
+    FlatWalk cw(n, RB);
+    for (int64_t c = cw.begin; c < cw.end; c += cw.stride) {
+      const int64_t e = c * RB + sub;
+      if (e >= n)
+        break;
+      const int64_t i = e * B + s;
+      const int2 ab = en_eff[e];
+      const double2 rv = csub(r[i], bil(alpha, w[i]));
+      r[i] = rv;
+      double2 z = bil(edge_diag_inv(e, s, P, k2, dK, dM, dMs, rport, coef), rv);
+      const bool hn = ab.x >= 0;
+      const double2 yd = csub(y[(int64_t)(hn ? ab.y : 0) * B + s], y[(int64_t)(hn ? ab.x : 0) * B + s]);
+      z = hn ? cadd(z, yd) : z;
+      v[0] = cadd(v[0], bil(rv, z));
+      v[1].x += cabs2(rv);
+    }
+  }
+  flat_partials<2>(v, red, partial, B, RB, sub, s);
+}
+
 // Frequency-independent diagonals: edge diagonals of K, M, Ms; nodal diag(G^T X G).
 __global__ void k_sw_edge_diag(int64_t n, const int32_t *__restrict__ row_ptr,
                                const int32_t *__restrict__ col, const double2 *__restrict__ K,
@@ -1786,12 +2089,14 @@ struct efm_sweep {
   // captured once per solve (after the autotuner has chosen the kernels)
   int use_graph = 0;
   hipStream_t capture_stream = nullptr;  // the chunk is captured here (a legacy null stream cannot capture)
+  int flat_blocks = 8;     // blocks of the narrow-batch kernels at most
   int gx_std[2] = {8, 8};  // grid of the standard form's update [VT c128, c64]
   // update grids (one block slice, as many blocks as are resident): [VT c128, c64][INIT, skip, apply]
   int gx_upd[2][3] = {{8, 8, 8}, {8, 8, 8}};
   float tune_ms[5] = {0.f, 0.f, 0.f, 0.f, 0.f};  // SpMV 0, 1, 2; nodal 0, 1
   efm::DevBuf K, M, Ms, rport, dK, dM, dMs, dnK, dnM, dnMs, gsign, en_eff;
   efm::DevBuf x, r, p, sv, u, w, y, part_u, part_s, state, flags, k0sq, coef;
+  efm::DevBuf KM, KMi;  // narrow batches: the values in pairs (made on first use)
   efm::DevBuf x64;  // reliable updates: FP64 solution (allocated on first use)
   efm::DevBuf dninv;  // [N][Bmax] inverse nodal diagonals of the systems of one solve
   efm::DevBuf tucol, tnu, tlidx, tdloc;  // row-tile format of the LDS-tiled SpMV
@@ -1897,6 +2202,8 @@ extern "C" int efm_sweep_create(const efm_topology *topo, const double *K_val, c
       gx_upd_max = std::max(gx_upd_max, s->gx_upd[a][b]);
     gx_upd_max = std::max(gx_upd_max, s->gx_std[a]);
   }
+  s->flat_blocks = std::max(8, ncu * 4 / 8 * 8);
+  gx_upd_max = std::max(gx_upd_max, s->flat_blocks);
   const int64_t ntl = (n + kTileRows - 1) / kTileRows;
   // K, M, Ms and the tile entry slots carry one zero entry at index nnz
   if ((rc = s->K.alloc((nnz + 1) * 16)) || (rc = s->M.alloc((nnz + 1) * 16)) ||
@@ -1911,7 +2218,7 @@ extern "C" int efm_sweep_create(const efm_topology *topo, const double *K_val, c
       (rc = s->y.alloc((size_t)N * s->Bmax * sizeof(double2))) ||
       (rc = s->dninv.alloc((size_t)N * s->Bmax * sizeof(double2))) ||
       (rc = s->part_u.alloc((size_t)groups * gx_upd_max * 2 * 64 * sizeof(double2))) ||
-      (rc = s->part_s.alloc((size_t)groups * std::max(std::max(s->gx_spmv, s->gx_pre), s->gx_tile) * 64 *
+      (rc = s->part_s.alloc((size_t)groups * std::max({s->gx_spmv, s->gx_pre, s->gx_tile, s->flat_blocks}) * 64 *
                             sizeof(double2))) ||
       (rc = s->state.alloc(s->Bmax * sizeof(SwState))) || (rc = s->flags.alloc(s->Bmax * sizeof(int))) ||
       (rc = s->k0sq.alloc(s->Bmax * sizeof(double))) ||
@@ -2193,6 +2500,14 @@ struct SwRun {
   int *flags;
   double2 *pu, *ps;
   std::vector<int> hflags;
+  bool flat = false;  // the narrow-batch kernels
+  FlatDims fd{};
+
+  // blocks of the narrow-batch kernels over `items` rows or nodes
+  int flat_gx(int64_t items) const {
+    const int64_t need = (items + fd.RB - 1) / fd.RB;
+    return (int)std::min<int64_t>(s->flat_blocks, (need + 7) / 8 * 8);
+  }
 
   int n_active(int &count) {
     int want = 0;
@@ -2214,7 +2529,15 @@ struct SwRun {
   // w = A_s u with SpMV variant `variant` (partials of u^T w in part_s)
   template <typename VT> int spmv_launch(int variant, const VT *u, VT *w) {
     const int64_t n = s->n;
-    if (variant == 2) {
+    if (variant == kFlatVariant) {
+      if constexpr (std::is_same<VT, double2>::value) {
+        auto k = s->cplx ? k_sf_spmv<true> : k_sf_spmv<false>;
+        const size_t lds = std::max<size_t>((size_t)(fd.stage + 1) * (s->cplx ? 36 : 20), (size_t)fd.T * 16);
+        hipLaunchKernelGGL(k, dim3(flat_gx(n)), dim3(fd.T), lds, st, n, Bp, fd.RB, fd.stage, P, s->row_ptr,
+                           s->col, s->KM.as<double2>(), s->KMi.as<double2>(), s->Ms.as<double>(),
+                           s->rport.as<int8_t>(), s->k0sq.as<double>(), s->coef.as<double2>(), u, w, ps, S);
+      }
+    } else if (variant == 2) {
       const dim3 grid(s->gx_tile, 1);
       const double2 *Kv = s->K.as<double2>(), *Mv = s->M.as<double2>(), *cf = s->coef.as<double2>();
       const double *Msv = s->Ms.as<double>(), *k2 = s->k0sq.as<double>();
@@ -2281,7 +2604,11 @@ struct SwRun {
   // y = Dn^{-1} G^T v with nodal variant `variant`, NV gathered vectors (see k_sw_aux_node)
   template <typename VT, int NV> int aux_launch(int variant, const VT *r, const VT *w, const VT *sv, VT *y) {
     const int8_t *gs = s->gsign.as<int8_t>();
-    if (variant == 1)
+    if (variant == kFlatVariant) {
+      if constexpr (std::is_same<VT, double2>::value && NV <= 2)
+        hipLaunchKernelGGL((k_sf_node<NV == 2>), dim3(flat_gx(s->N)), dim3(fd.T), (size_t)fd.stage * 8, st,
+                           s->N, Bp, fd.RB, fd.stage, s->n2e_ptr, s->n2e, gs, s->dninv.as<double2>(), r, w, y, S);
+    } else if (variant == 1)
       hipLaunchKernelGGL((k_sw_aux_pre<VT, NV>), dim3(s->gx_aux, 1), dim3(kBlock), 0, st, s->N, Bp, groups,
                          s->n2e_ptr, s->n2e, gs, s->dninv.as<double2>(), r, w, sv, y, S);
     else
@@ -2481,18 +2808,24 @@ struct SwRun {
     auto fin = [&](auto stage, int gx, const double2 *part) -> int {
       constexpr int STAGE = decltype(stage)::value;
       const bool corr = STAGE == 1 && s->c_rows > 0;
-      hipLaunchKernelGGL((k_sw_fin_std<STAGE>), dim3(Bp), dim3(kBlock), 0, st, Bp, gx, part, corr ? s->gx_corr : 0,
+      hipLaunchKernelGGL((k_sw_fin_std<STAGE>), dim3((Bp + 7) / 8 * 8), dim3(kBlock), 0, st, Bp, gx, part, corr ? s->gx_corr : 0,
                          corr ? (const double2 *)s->part_c.as<double2>() : (const double2 *)nullptr, S, flags,
                          inner_tol2, max_it, max_inner, ru_delta2);
       EFM_LAUNCH_CHECK();
       return EFM_OK;
     };
-    auto gxs_of = [&](int v) { return v == 2 ? s->gx_tile : v == 1 ? s->gx_pre : s->gx_spmv; };
-    // autotuning in place, as in cocg()
+    auto gxs_of = [&](int v) {
+      return v == kFlatVariant ? flat_gx(n) : v == 2 ? s->gx_tile : v == 1 ? s->gx_pre : s->gx_spmv;
+    };
+    // autotuning in place, as in cocg() (nothing to choose for a narrow batch)
     const int nvs = s->tiled_ok ? 3 : 2;
     TuneLog log_s, log_a;
-    auto vs_of = [&](int it) { return s->spmv_variant >= 0 ? s->spmv_variant : it % nvs; };
-    auto va_of = [&](int it) { return s->aux_variant >= 0 ? s->aux_variant : (it >= 0 ? it % 2 : 1); };
+    const int sv0 = flat ? kFlatVariant : s->spmv_variant, av0 = flat ? kFlatVariant : s->aux_variant;
+    const bool tune_s = sv0 < 0, tune_a = av0 < 0;
+    auto vs_of = [&](int it) { return !tune_s ? sv0 : s->spmv_variant >= 0 ? s->spmv_variant : it % nvs; };
+    auto va_of = [&](int it) {
+      return !tune_a ? av0 : s->aux_variant >= 0 ? s->aux_variant : (it >= 0 ? it % 2 : 1);
+    };
     auto run = [&](TuneLog &lg, bool timed, int v, auto &&launch) -> int {
       if (!timed)
         return launch();
@@ -2509,6 +2842,18 @@ struct SwRun {
         return rc2;
       EFM_HIP_CHECK(hipEventRecord(e1, st));
       return EFM_OK;
+    };
+    auto vs_timed = [&]() { return tune_s && s->spmv_variant < 0; };
+    auto va_timed = [&]() { return tune_a && s->aux_variant < 0; };
+    auto launch_flat_p = [&]() {
+      if constexpr (std::is_same<VT, double2>::value)
+        hipLaunchKernelGGL(k_sf_pform, dim3(flat_gx(n)), dim3(fd.T), 0, st, n, Bp, fd.RB, P, en, dK,
+                           dM, dMs, rp, k2, cf, y, r, p, x, S);
+    };
+    auto launch_flat_r = [&]() {
+      if constexpr (std::is_same<VT, double2>::value)
+        hipLaunchKernelGGL(k_sf_update, dim3(flat_gx(n)), dim3(fd.T), 0, st, n, Bp, fd.RB, P, en,
+                           dK, dM, dMs, rp, k2, cf, y, w, r, pu, S);
     };
     // u = P r, rho = u^T r
     int rc, active = 0;
@@ -2531,7 +2876,8 @@ struct SwRun {
       }
       const int chunk = std::min(check, cap - it);
       // a full chunk with the kernels chosen: replay the captured graph (capture it first)
-      const bool replay = s->use_graph && chunk == check && s->spmv_variant >= 0 && s->aux_variant >= 0;
+      const bool replay =
+          s->use_graph && chunk == check && (flat || (s->spmv_variant >= 0 && s->aux_variant >= 0));
       if (replay && graph.x) {
         EFM_HIP_CHECK(hipGraphLaunch(graph.x, st));
         it += chunk;
@@ -2554,7 +2900,9 @@ struct SwRun {
       }
       for (int c = 0; c < chunk; ++c, ++it) {
         const int va = va_of(it), vs = vs_of(it);
-        if (s->form == 2 && xlag)
+        if (flat)
+          launch_flat_p();
+        else if (s->form == 2 && xlag)
           hipLaunchKernelGGL((k_sw_pform_u<VT, true>), dim3(s->gx_vec, groups), dim3(kBlock), 0, st, n, Bp, P, en,
                              dK, dM, dMs, rp, k2, cf, (const VT *)y, (const VT *)r, p, x, S);
         else if (s->form == 2)
@@ -2564,17 +2912,20 @@ struct SwRun {
           hipLaunchKernelGGL((k_sw_pform<VT>), dim3(s->gx_vec, groups), dim3(kBlock), 0, st, n, Bp, (const VT *)u,
                              p, S);
         EFM_LAUNCH_CHECK();
-        if ((rc = run(log_s, s->spmv_variant < 0, vs, [&]() { return spmv_launch<VT>(vs, p, w); })) ||
+        if ((rc = run(log_s, vs_timed(), vs, [&]() { return spmv_launch<VT>(vs, p, w); })) ||
             (rc = fin(std::integral_constant<int, 1>{}, gxs_of(vs), ps)) ||
-            (rc = run(log_a, s->aux_variant < 0, va,
+            (rc = run(log_a, va_timed(), va,
                       [&]() { return aux_launch<VT, 2>(va, r, w, (const VT *)nullptr, y); })))
           return rc;
         auto upd = s->form != 2 ? k_sw_update_std<VT, true, false>
                                 : xlag ? k_sw_update_std<VT, false, true> : k_sw_update_std<VT, false, false>;
-        hipLaunchKernelGGL(upd, dim3(s->gx_std[vti], 1), dim3(kBlock), 0, st, n, Bp, groups, P, en, dK, dM, dMs,
-                           rp, k2, cf, (const VT *)y, (const VT *)w, (const VT *)p, u, x, r, pu, S);
+        if (flat)
+          launch_flat_r();
+        else
+          hipLaunchKernelGGL(upd, dim3(s->gx_std[vti], 1), dim3(kBlock), 0, st, n, Bp, groups, P, en, dK, dM, dMs,
+                             rp, k2, cf, (const VT *)y, (const VT *)w, (const VT *)p, u, x, r, pu, S);
         EFM_LAUNCH_CHECK();
-        if ((rc = fin(std::integral_constant<int, 2>{}, s->gx_std[vti], pu)))
+        if ((rc = fin(std::integral_constant<int, 2>{}, flat ? flat_gx(n) : s->gx_std[vti], pu)))
           return rc;
       }
       if (replay) {  // the chunk was captured, not run: instantiate and launch it
@@ -2630,7 +2981,9 @@ extern "C" int efm_sweep_solve(efm_sweep *s, int nsys, const double *h_k0sq, con
   EFM_REQUIRE(s->c_rows == 0 || ((s->c_vals || s->c_nnz == 0) && s->c_nsys == nsys),
               "efm_sweep_solve: correction values missing or set for another number of systems");
   hipStream_t st = (hipStream_t)stream;
-  const int Bp = ((nsys + kSys - 1) / kSys) * kSys;  // padded system count this call
+  const bool flat = !h_refine && s->form == 2 && s->spmv_variant < 0 && s->aux_variant < 0 && flat_wins(s->n, nsys);
+  // the wide kernels' system count is padded to whole wavefronts
+  const int Bp = flat ? nsys : ((nsys + kSys - 1) / kSys) * kSys;
   const int P = s->P;
   // per-system scalars (padding systems get zero right-hand sides and stay inactive)
   std::vector<double> k2(Bp, 0.0);
@@ -2658,7 +3011,19 @@ extern "C" int efm_sweep_solve(efm_sweep *s, int nsys, const double *h_k0sq, con
   run.s = s;
   run.st = st;
   run.Bp = Bp;
-  run.groups = Bp / kSys;
+  run.groups = (Bp + kSys - 1) / kSys;
+  run.flat = flat;
+  if (flat) {
+    run.fd = flat_dims(nsys);
+    if (!s->KM.p) {
+      int rc2;
+      if ((rc2 = s->KM.alloc((size_t)s->nnz * 16)) || (s->cplx && (rc2 = s->KMi.alloc((size_t)s->nnz * 16))))
+        return rc2;
+      hipLaunchKernelGGL(k_sf_pair, dim3(grid_for(s->nnz, 256)), dim3(256), 0, st, s->nnz, s->K.as<double2>(),
+                         s->M.as<double2>(), s->KM.as<double2>(), s->KMi.as<double2>());
+      EFM_LAUNCH_CHECK();
+    }
+  }
   run.P = P;
   run.check = h_opts->check_every > 0 ? h_opts->check_every : 16;
   run.tol2 = h_opts->tolerance * h_opts->tolerance;

@@ -192,14 +192,12 @@ int efm_solver_solve(efm_solver *s, const double *B, double *X, const efm_solve_
  * length inside windows of 4096, no LDS; built on the device at first use); 11: variant 9
  * with the values stored as a real part per entry plus the imaginary parts of the tiles
  * that have any (a tile of real values streams 8 B per value instead of 16; complex-double
- * matrices; rebuilt on the device after every set_matrix); 12: all iterations in one
- * persistent kernel that keeps the matrix in registers and LDS, COCG on complex-double
- * matrices of up to 512 rows per CU (256 with three or four right-hand sides) whose blocks of
- * rows read few enough columns, with at most four low-rank terms times right-hand sides;
- * a solve that it does not cover is refused).  By default (-1) systems that variant 12
- * covers are solved with it (get reports -1); for others the first solve times variants
- * 0-11 on the installed matrix and keeps the fastest; a fixed variant makes results
- * reproducible bit for bit across runs.
+ * matrices; rebuilt on the device after every set_matrix).  By
+ * default (-1) complex-double COCG solves of up to 512 rows per CU (256 with three or four
+ * right-hand sides; at most four low-rank terms times right-hand sides) run in one
+ * persistent kernel that keeps the matrix in registers and LDS (get reports -1); for
+ * others the first solve times variants 0-11 on the installed matrix and keeps the
+ * fastest; a fixed variant makes results reproducible bit for bit across runs.
  * h_tune_ms (12 entries, may be NULL) receives the
  * measured average ms per launch (-1 = not available).  No reference counterpart. */
 int efm_solver_set_spmv_variant(efm_solver *s, int variant);
@@ -295,8 +293,10 @@ int efm_sweep_solve(efm_sweep *sw, int nsys, const double *h_k0sq, const double 
  * that each XCD's share of the gathered vectors stays in its L2); 2 (SpMV only) =
  * LDS-tiled: each tile of 8 consecutive rows loads its distinct columns (at most 72)
  * once per group of 64 systems into LDS and its rows read them there; available when
- * every tile fits (set returns an error otherwise); -1 (default) = the fastest, chosen on
- * the first solve: the iterations before its first convergence check cycle through the
+ * every tile fits (set returns an error otherwise); -1 (default) = with form 2, no
+ * reliable updates and a batch that would leave many of its wavefronts' lanes idle (below
+ * 40, 65-95 and 129-143 systems), kernels that pack the systems of several rows into a wavefront (get reports -1);
+ * otherwise the fastest, chosen on the first solve: the iterations before its first convergence check cycle through the
  * candidates, each launch timed in place.  get: the variants in use (-1 before they are
  * chosen) and, when h_tune_ms is given (5 entries), the mean times in ms per launch
  * [SpMV 0, 1, 2, nodal 0, 1] (0 for a variant not timed).  Autotuner of this project; no
