@@ -20,6 +20,7 @@
 // `check_every` iterations.
 #include "efm_internal.h"
 #include "efm_persist.h"
+#include "efm_staged.h"
 
 #include <algorithm>
 #include <climits>
@@ -1787,6 +1788,13 @@ struct efm_solver {
   efm::DevBuf sp_re, sp_im, sp_off;
   int64_t sp_im_n = 0;
   bool sp_ok = false;
+  // variant 11 with one or two right-hand sides: tiles whose columns are staged in LDS
+  // (efm_staged.h), built on first use, the values after every set_matrix
+  efm::DevBuf st_srow, st_sown, st_steps, st_ucol, st_nu, st_idx, st_re, st_im, st_iflag;
+  int st_state = 0;  // 0: not tried, 1: built, -1: a tile does not fit
+  int st_ntiles = 0, st_cap = 0, st_lds = 0;
+  int64_t st_pairs = 0;
+  bool st_vals_ok = false;
   int grid_rows[3] = {8, 8, 8};
   int spmv_variant = -1;  // -1: choose by timing at the first solve
   double tune_ms[kNumSpmvVariants] = {0};
@@ -2008,6 +2016,103 @@ template <int R> struct Dispatch {
     return EFM_OK;
   }
 
+  static void drop_staged(efm_solver *s) {
+    for (DevBuf *b : {&s->st_srow, &s->st_sown, &s->st_steps, &s->st_ucol, &s->st_nu, &s->st_idx, &s->st_re, &s->st_im,
+                      &s->st_iflag})
+      (void)b->alloc(0);
+    s->st_state = -1;
+  }
+  // The staged tiles of variant 11: structure once, values after every set_matrix.
+  // s->st_state < 0: a tile does not fit, or there is no room.
+  static int build_staged(efm_solver *s, hipStream_t st) {
+    using namespace efm_staged;
+    const int64_t n = s->n;
+    if (s->st_state == 0) {
+      s->st_state = -1;
+      const int64_t nt = (n + kTile - 1) / kTile, nw = nt * kWavesT;
+      const int cap = std::min<int64_t>(kMaxLds / (16 * R), 0x10000);
+      if (n * R >= INT32_MAX || (nt + 7) / 8 * 8 * R * sizeof(double2) > s->partial.bytes)
+        return EFM_OK;
+      DevBuf pairs, window, bad;
+      if (pairs.alloc((size_t)nw * 4) || window.alloc((size_t)nt * sizeof(int2)) || bad.alloc(sizeof(int)) ||
+          s->st_srow.alloc((size_t)nt * kTile * 2))
+        return EFM_OK;
+      EFM_HIP_CHECK(hipMemsetAsync(bad.p, 0, sizeof(int), st));
+      hipLaunchKernelGGL(k_order, dim3((unsigned)nt), dim3(kTile), 0, st, (int)n, s->row_ptr, s->col,
+                         s->st_srow.as<uint16_t>(), pairs.as<int32_t>(), window.as<int2>(), bad.as<int>());
+      EFM_LAUNCH_CHECK();
+      std::vector<int32_t> hp(nw);
+      std::vector<int2> hw(nt), steps(nw);
+      int hbad = 0;
+      EFM_HIP_CHECK(hipMemcpyAsync(hp.data(), pairs.p, nw * 4, hipMemcpyDeviceToHost, st));
+      EFM_HIP_CHECK(hipMemcpyAsync(hw.data(), window.p, nt * sizeof(int2), hipMemcpyDeviceToHost, st));
+      EFM_HIP_CHECK(hipMemcpyAsync(&hbad, bad.p, sizeof(int), hipMemcpyDeviceToHost, st));
+      EFM_HIP_CHECK(hipStreamSynchronize(st));
+      int64_t total = 0;
+      for (int64_t i = 0; i < nw; ++i) {
+        steps[i] = make_int2((int)total, hp[i]);
+        total += hp[i];
+      }
+      int words = 0;
+      for (const int2 &w : hw)
+        words = std::max(words, (w.y - (w.x & ~31)) / 32 + 1);
+      if (hbad || words > kMaxWords || total >= INT32_MAX)
+        return EFM_OK;
+      // one step more than is stored: a wavefront without rows at the end reads it, unused
+      if (s->st_steps.alloc((size_t)nw * sizeof(int2)) || s->st_sown.alloc((size_t)nt * kTile * 2) ||
+          s->st_ucol.alloc((size_t)nt * cap * 4) || s->st_nu.alloc((size_t)nt * 4) ||
+          s->st_idx.alloc((size_t)(total + 1) * 64 * 4) || s->st_iflag.alloc((size_t)nt * 4) ||
+          s->st_re.alloc((size_t)(total + 1) * 64 * 16)) {
+        drop_staged(s);  // no room: the split values as before
+        return EFM_OK;
+      }
+      EFM_HIP_CHECK(hipMemcpyAsync(s->st_steps.p, steps.data(), nw * sizeof(int2), hipMemcpyHostToDevice, st));
+      const void *k = reinterpret_cast<const void *>(&k_index);
+      EFM_HIP_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, words * 8));
+      hipLaunchKernelGGL(k_index, dim3((unsigned)nt), dim3(kTile), words * 8, st, (int)n, words, cap, s->row_ptr,
+                         s->col, s->st_srow.as<uint16_t>(), s->st_steps.as<int2>(), window.as<int2>(),
+                         s->st_ucol.as<int32_t>(), s->st_nu.as<int32_t>(), s->st_sown.as<uint16_t>(),
+                         s->st_idx.as<uint32_t>());
+      EFM_LAUNCH_CHECK();
+      std::vector<int32_t> nu(nt);
+      EFM_HIP_CHECK(hipMemcpyAsync(nu.data(), s->st_nu.p, nt * 4, hipMemcpyDeviceToHost, st));
+      EFM_HIP_CHECK(hipStreamSynchronize(st));
+      if (*std::min_element(nu.begin(), nu.end()) < 0) {
+        drop_staged(s);
+        return EFM_OK;
+      }
+      s->st_ntiles = (int)nt;
+      s->st_cap = cap;
+      s->st_lds = *std::max_element(nu.begin(), nu.end()) * R * (int)sizeof(double2);
+      s->st_pairs = total;
+      EFM_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&efm_staged::k_staged<R, SysState>),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, s->st_lds));
+      s->st_state = 1;
+    }
+    if (s->st_state < 0)
+      return EFM_OK;
+    // the imaginary array is made when a matrix has imaginary parts
+    for (int pass = 0; pass < 2; ++pass) {
+      hipLaunchKernelGGL(k_values, dim3((unsigned)s->st_ntiles), dim3(kTile), 0, st, (int)n, s->row_ptr,
+                         s->val.as<double2>(), s->st_srow.as<uint16_t>(), s->st_steps.as<int2>(),
+                         s->st_re.as<double2>(), s->st_im.as<double2>(), s->st_iflag.as<int>());
+      EFM_LAUNCH_CHECK();
+      if (s->st_im.p)
+        break;
+      std::vector<int> fl(s->st_ntiles);
+      EFM_HIP_CHECK(hipMemcpyAsync(fl.data(), s->st_iflag.p, fl.size() * 4, hipMemcpyDeviceToHost, st));
+      EFM_HIP_CHECK(hipStreamSynchronize(st));
+      if (*std::max_element(fl.begin(), fl.end()) == 0)
+        break;
+      if (s->st_im.alloc((size_t)(s->st_pairs + 1) * 64 * 16)) {
+        drop_staged(s);
+        return EFM_OK;
+      }
+    }
+    s->st_vals_ok = true;
+    return EFM_OK;
+  }
+
   // One fused SpMV of the given variant; *nb = number of partial sums written.
   template <typename VT>
   static int launch_spmv(efm_solver *s, int variant, const double2 *Wa, double2 *Wb, hipStream_t st,
@@ -2074,6 +2179,22 @@ template <int R> struct Dispatch {
     case kSplitForm:
       if constexpr (std::is_same<VT, double2>::value) {
         int rc;
+        if constexpr (R <= 2) {
+          if (s->st_state >= 0 && !s->st_vals_ok && (rc = build_staged(s, st)) != EFM_OK)
+            return rc;
+          if (s->st_state > 0) {
+            const int span = (s->st_ntiles + 7) / 8;
+            *nb = 8 * span;
+            auto k = &efm_staged::k_staged<R, SysState>;
+            hipLaunchKernelGGL(k, dim3(*nb), dim3(efm_staged::kTile), s->st_lds, st, (int)s->n, s->st_ntiles, span,
+                               s->st_cap, s->st_steps.as<int2>(), s->st_srow.as<uint16_t>(),
+                               s->st_sown.as<uint16_t>(), s->st_ucol.as<int32_t>(), s->st_nu.as<int32_t>(),
+                               s->st_idx.as<uint32_t>(), s->st_re.as<double2>(), s->st_im.as<double2>(),
+                               s->st_iflag.as<int>(), s->pf.as<double2>(), s->q.as<double2>(),
+                               s->partial.as<double2>(), S);
+            break;
+          }
+        }
         if (!s->sp_ok && (rc = build_split(s, st)) != EFM_OK)
           return rc;
         *nb = s->grid_z;
@@ -2636,6 +2757,7 @@ extern "C" int efm_solver_set_matrix(efm_solver *s, const void *values, void *st
   EFM_HIP_CHECK(hipMemcpyAsync(s->val.p, values, s->val.bytes, hipMemcpyDeviceToDevice, st));
   s->sell_vals_ok = false;  // the sliced-ELL values are refilled at the next SpMV of variant 10
   s->sp_ok = false;         // and the split values of variant 11 rebuilt
+  s->st_vals_ok = false;
   if (s->vtype == EFM_C128)
     hipLaunchKernelGGL(k_dinv<double2>, dim3(grid_for(s->n, 256)), dim3(256), 0, st, s->n, s->row_ptr,
                        s->col, s->val.as<double2>(), s->dinv.as<double2>());

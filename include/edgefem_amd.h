@@ -192,7 +192,8 @@ int efm_solver_solve(efm_solver *s, const double *B, double *X, const efm_solve_
  * length inside windows of 4096, no LDS; built on the device at first use); 11: variant 9
  * with the values stored as a real part per entry plus the imaginary parts of the tiles
  * that have any (a tile of real values streams 8 B per value instead of 16; complex-double
- * matrices; rebuilt on the device after every set_matrix).  By
+ * matrices; rebuilt on the device after every set_matrix), and, with one or two right-hand
+ * sides where the columns of every 512 rows fit, those columns staged in LDS.  By
  * default (-1) complex-double COCG solves of up to 512 rows per CU (256 with three or four
  * right-hand sides; at most four low-rank terms times right-hand sides) run in one
  * persistent kernel that keeps the matrix in registers and LDS (get reports -1); for

@@ -224,3 +224,52 @@ def test_packed_sweep_batches(torch_dev, nsys, levels, ring, lossy, graph):
     print(f"n {n} nsys {nsys}: iterations {iters.max()} true {rel:.1e}; 5 iterations against padded {d:.1e}", flush=True)
     assert iters.max() < 200 and rel <= 2e-10 and np.all(Y[:, ~on] == 0)
     assert d <= 1e-9
+
+
+@pytest.mark.parametrize("n,nrhs,kind", [
+    (5, 1, "real"), (511, 2, "mixed"), (512, 1, "complex"), (513, 2, "real"), (1600, 2, "mixed"), (9000, 1, "mixed"),
+    (40000, 2, "scattered"), (3000, 2, "long")])
+def test_staged_spmv_tiles(torch_dev, n, nrhs, kind):
+    """SpMV variant 11 with tiles of 512 rows: a last tile of one row, wavefronts without rows,
+    real and complex tiles side by side, rows of 250 entries, columns that do not fit (then
+    without staging); a second matrix on the same solver.  True residual as in
+    test_persistent_cocg_edges; 7 iterations against one launch per row group likewise."""
+    import scipy.sparse as sp
+    import torch
+    from edgefem_amd import _capi
+    A, en, B = _local_system(n, nrhs, n + 1, long_rows=(0, n // 2, n - 1))
+    rng = np.random.default_rng(n)
+    if kind == "scattered":
+        perm = rng.permutation(n)
+        A = A[perm][:, perm].tocsr()
+    elif kind == "long":
+        j = np.arange(n // 2 + 1, n // 2 + 225)
+        far = sp.csr_matrix((np.full(j.size, 0.01 + 0.01j), (np.full(j.size, n // 2), j)), shape=(n, n))
+        A = (A + far + far.T + 6 * sp.identity(n)).tocsr()
+    A.sort_indices()
+    mats = [A]
+    if kind in ("real", "mixed"):
+        half = n if kind == "real" else n // 2
+        Ar = A.copy()
+        row = np.repeat(np.arange(n), np.diff(A.indptr))
+        Ar.data = np.where((row < half) & (A.indices < half), np.abs(A.data.real) * np.sign(A.data.real), A.data)
+        Ar = (Ar + sp.diags(np.asarray(abs(A).sum(axis=1)).ravel())).tocsr()
+        Ar.sort_indices()
+        mats = [Ar, A] if kind == "mixed" else [Ar]
+    s = _capi.KrylovSolver(A.indptr, A.indices, nrhs=nrhs)
+    s.set_gradient(_Nodes(en))
+    b = torch.from_numpy(B).cuda()
+    for Am in mats:
+        assert np.array_equal(Am.indices, A.indices)
+        s.set_matrix(Am.data)
+        X = {}
+        for variant, cap in ((11, 1000), (11, 7), (0, 7)):
+            s.set_spmv_variant(variant)
+            X[variant, cap], info = s.solve(b, tol=1e-12, max_iterations=cap)
+            X[variant, cap] = X[variant, cap].cpu().numpy().reshape(n, nrhs)
+            if cap == 1000:
+                rel = (np.linalg.norm(B - Am @ X[variant, cap], axis=0) / np.linalg.norm(B, axis=0)).max()
+                print(f"n {n} {kind}: iterations {max(info['iters'])} true {rel:.1e}", flush=True)
+                assert info["converged"] and rel <= 2e-12
+        d = np.abs(X[11, 7] - X[0, 7]).max() / np.abs(X[0, 7]).max()
+        assert d <= max(1e-13, n * 2.3e-16), d
