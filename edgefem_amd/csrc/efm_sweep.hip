@@ -1976,45 +1976,59 @@ __device__ inline int gsign_of(const int32_t *__restrict__ en, int32_t e, int32_
 }
 
 // one thread per node: diag(G^T X G) for X in {K, M, Ms_p} (Dirichlet edges dropped)
-__global__ void k_sw_node_diag(int64_t N, int P, const int32_t *__restrict__ n2e_ptr,
-                               const int32_t *__restrict__ n2e, const int32_t *__restrict__ en,
-                               const uint8_t *__restrict__ dir, const int32_t *__restrict__ row_ptr,
-                               const int32_t *__restrict__ col, const double2 *__restrict__ K,
-                               const double2 *__restrict__ M, const double *const *__restrict__ Msp,
-                               double2 *__restrict__ dnK, double2 *__restrict__ dnM,
-                               double *__restrict__ dnMs) {
-  int64_t nd = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (nd >= N)
-    return;
+// kDiagLanes lanes per node, one incident edge per lane at a time: 39 us (one thread per node 261
+// us) for 7 k nodes.
+constexpr int kDiagLanes = 16;
+__global__ void __launch_bounds__(kBlock)
+    k_sw_node_diag(int64_t N, int P, const int32_t *__restrict__ n2e_ptr, const int32_t *__restrict__ n2e,
+                   const int32_t *__restrict__ en, const uint8_t *__restrict__ dir,
+                   const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col,
+                   const double2 *__restrict__ K, const double2 *__restrict__ M,
+                   const double *const *__restrict__ Msp, double2 *__restrict__ dnK, double2 *__restrict__ dnM,
+                   double *__restrict__ dnMs) {
+  const int64_t nd = ((int64_t)blockIdx.x * kBlock + threadIdx.x) / kDiagLanes;
+  const int l = threadIdx.x % kDiagLanes;
   double2 sk = make_double2(0, 0), sm = make_double2(0, 0);
-  double sp[kMaxPorts] = {0, 0, 0, 0};
-  for (int32_t k = n2e_ptr[nd]; k < n2e_ptr[nd + 1]; ++k) {
-    const int32_t e = n2e[k];
-    if (dir && dir[e])
-      continue;
-    const int ge = gsign_of(en, e, (int32_t)nd);
-    if (!ge)
-      continue;
-    for (int32_t q = row_ptr[e]; q < row_ptr[e + 1]; ++q) {
-      const int32_t f = col[q];
-      if (dir && dir[f])
+  double2 sp[kMaxPorts / 2];
+  for (int p = 0; p < kMaxPorts / 2; ++p)
+    sp[p] = make_double2(0, 0);
+  if (nd < N)
+    for (int32_t k = n2e_ptr[nd] + l; k < n2e_ptr[nd + 1]; k += kDiagLanes) {
+      const int32_t e = n2e[k];
+      const int ge = dir && dir[e] ? 0 : gsign_of(en, e, (int32_t)nd);
+      if (!ge)
         continue;
-      const int gf = gsign_of(en, f, (int32_t)nd);
-      if (!gf)
-        continue;
-      const double sg = (double)(ge * gf);
-      sk.x += sg * K[q].x;
-      sk.y += sg * K[q].y;
-      sm.x += sg * M[q].x;
-      sm.y += sg * M[q].y;
-      for (int p = 0; p < P; ++p)
-        sp[p] += sg * Msp[p][q];
+#pragma unroll 4
+      for (int32_t q = row_ptr[e]; q < row_ptr[e + 1]; ++q) {
+        const int32_t f = col[q];
+        const int gf = dir && dir[f] ? 0 : gsign_of(en, f, (int32_t)nd);
+        if (gf) {
+          const double sg = (double)(ge * gf);
+          const double2 kv = K[q], mv = M[q];
+          sk.x += sg * kv.x;
+          sk.y += sg * kv.y;
+          sm.x += sg * mv.x;
+          sm.y += sg * mv.y;
+#pragma unroll
+          for (int p = 0; p < kMaxPorts; ++p)
+            if (p < P)
+              (p & 1 ? sp[p / 2].y : sp[p / 2].x) += sg * Msp[p][q];
+        }
+      }
     }
-  }
+  group_sum<kDiagLanes>(sk);
+  group_sum<kDiagLanes>(sm);
+#pragma unroll
+  for (int p = 0; p < kMaxPorts / 2; ++p)
+    group_sum<kDiagLanes>(sp[p]);
+  if (nd >= N || l != 0)
+    return;
   dnK[nd] = sk;
   dnM[nd] = sm;
-  for (int p = 0; p < P; ++p)
-    dnMs[(int64_t)p * N + nd] = sp[p];
+#pragma unroll
+  for (int p = 0; p < kMaxPorts; ++p)
+    if (p < P)
+      dnMs[(int64_t)p * N + nd] = p & 1 ? sp[p / 2].y : sp[p / 2].x;
 }
 
 __global__ void k_sw_gsign(int64_t N, const int32_t *__restrict__ n2e_ptr, const int32_t *__restrict__ n2e,
@@ -2247,7 +2261,7 @@ extern "C" int efm_sweep_create(const efm_topology *topo, const double *K_val, c
                      s->dM.as<double2>(), s->dMs.as<double>());
   EFM_LAUNCH_CHECK();
   const int32_t *en = topo->edge_nidx.as<int32_t>();
-  hipLaunchKernelGGL(k_sw_node_diag, dim3(grid_for(N, 256)), dim3(256), 0, st, N, n_ports, s->n2e_ptr,
+  hipLaunchKernelGGL(k_sw_node_diag, dim3(grid_for(N * kDiagLanes, kBlock)), dim3(kBlock), 0, st, N, n_ports, s->n2e_ptr,
                      s->n2e, en, dirichlet, s->row_ptr, s->col, s->K.as<double2>(), s->M.as<double2>(),
                      (const double *const *)ptab.p, s->dnK.as<double2>(), s->dnM.as<double2>(),
                      s->dnMs.as<double>());
