@@ -251,13 +251,53 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
-int element_blocks(const efm_topology *topo, const double *xyz, hipStream_t st, DevBuf &km) {
-  int rc = km.alloc((size_t)topo->T * 21 * sizeof(double2) + 16);
+// The scratch of one assembly: the topology's, or its own where another call holds that.  The
+// work that uses it has ended when it is given back.
+struct ElementScratch {
+  const efm_topology *topo;
+  hipStream_t st;
+  DevBuf own;
+  bool kept = false, idle = false;
+  ElementScratch(const efm_topology *t, hipStream_t s) : topo(t), st(s) {}
+  ~ElementScratch() {
+    if (!idle)
+      (void)hipStreamSynchronize(st);
+    if (kept) {
+      std::lock_guard<std::mutex> g(topo->km_lock);
+      topo->km_held = false;
+    }
+  }
+  int get(double2 **out) {
+    const size_t bytes = (size_t)topo->T * 21 * sizeof(double2) + 16;
+    std::lock_guard<std::mutex> g(topo->km_lock);
+    kept = !topo->km_held;
+    DevBuf &b = kept ? topo->km : own;
+    if (!b.p) {
+      const int rc = b.alloc(bytes);
+      if (rc != EFM_OK) {
+        kept = false;
+        return rc;
+      }
+    }
+    if (kept)
+      topo->km_held = true;
+    *out = b.as<double2>();
+    return EFM_OK;
+  }
+  int wait() {
+    EFM_HIP_CHECK(hipStreamSynchronize(st));
+    idle = true;
+    return EFM_OK;
+  }
+};
+
+int element_blocks(const efm_topology *topo, const double *xyz, hipStream_t st, ElementScratch &scratch,
+                   double2 **km) {
+  int rc = scratch.get(km);
   if (rc != EFM_OK)
     return rc;
   hipLaunchKernelGGL(k_element_blocks, dim3(grid_for(topo->T, kBlock)), dim3(kBlock), 0, st,
-                     topo->T, topo->tet_nodes.as<int32_t>(), xyz, topo->tet_sign.as<int8_t>(),
-                     km.as<double2>());
+                     topo->T, topo->tet_nodes.as<int32_t>(), xyz, topo->tet_sign.as<int8_t>(), *km);
   EFM_LAUNCH_CHECK();
   return EFM_OK;
 }
@@ -269,18 +309,18 @@ extern "C" int efm_assemble_km(const efm_topology *topo, const double *xyz, cons
                                double *M_val, void *stream) {
   EFM_REQUIRE(topo && xyz && eps_tet && K_val && M_val, "efm_assemble_km: NULL argument");
   hipStream_t st = (hipStream_t)stream;
-  DevBuf km;
-  int rc = element_blocks(topo, xyz, st, km);
+  ElementScratch scratch(topo, st);
+  double2 *km = nullptr;
+  int rc = element_blocks(topo, xyz, st, scratch, &km);
   if (rc != EFM_OK)
     return rc;
   hipLaunchKernelGGL(k_gather_km, dim3(grid_for(topo->nnz, kBlock)), dim3(kBlock), 0, st,
                      topo->nnz, topo->row_idx.as<int32_t>(), topo->col_idx.as<int32_t>(),
-                     topo->cptr.as<int32_t>(), topo->contrib.as<int32_t>(), km.as<double2>(),
+                     topo->cptr.as<int32_t>(), topo->contrib.as<int32_t>(), km,
                      (const double2 *)eps_tet, (const double2 *)inv_mu_tet, dirichlet,
                      (double2 *)K_val, (double2 *)M_val);
   EFM_LAUNCH_CHECK();
-  EFM_HIP_CHECK(hipStreamSynchronize(st));  // scratch is freed on return
-  return EFM_OK;
+  return scratch.wait();
 }
 
 extern "C" int efm_assemble_maxwell(const efm_topology *topo, const double *xyz,
@@ -289,19 +329,19 @@ extern "C" int efm_assemble_maxwell(const efm_topology *topo, const double *xyz,
                                     double omega, double *A_val, void *stream) {
   EFM_REQUIRE(topo && xyz && eps_tet && A_val, "efm_assemble_maxwell: NULL argument");
   hipStream_t st = (hipStream_t)stream;
-  DevBuf km;
-  int rc = element_blocks(topo, xyz, st, km);
+  ElementScratch scratch(topo, st);
+  double2 *km = nullptr;
+  int rc = element_blocks(topo, xyz, st, scratch, &km);
   if (rc != EFM_OK)
     return rc;
   const double k0 = omega / kC0;
   hipLaunchKernelGGL(k_gather_a, dim3(grid_for(topo->nnz, kBlock)), dim3(kBlock), 0, st, topo->nnz,
                      topo->row_idx.as<int32_t>(), topo->col_idx.as<int32_t>(),
-                     topo->cptr.as<int32_t>(), topo->contrib.as<int32_t>(), km.as<double2>(),
+                     topo->cptr.as<int32_t>(), topo->contrib.as<int32_t>(), km,
                      (const double2 *)eps_tet, (const double2 *)inv_mu_tet, dirichlet, abc_mask,
                      k0, (double2 *)A_val);
   EFM_LAUNCH_CHECK();
-  EFM_HIP_CHECK(hipStreamSynchronize(st));
-  return EFM_OK;
+  return scratch.wait();
 }
 
 extern "C" int efm_port_surface_mass(const efm_topology *topo, const double *xyz, int64_t n_sel,

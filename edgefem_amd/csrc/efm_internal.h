@@ -3,6 +3,8 @@
 
 #include "efm_common.h"
 
+#include <mutex>
+
 namespace efm {
 
 size_t scan_work_bytes(int64_t n);
@@ -63,4 +65,10 @@ struct efm_topology {
   efm::DevBuf edge_nidx;  // int32 [2*n_edges] node positions (lower-ID end, higher-ID end)
   efm::DevBuf n2e_ptr;    // int32 [N+1]   node -> incident edges, ascending
   efm::DevBuf n2e;        // int32 [2*n_edges]
+  // element blocks of an assembly (336 B per tet), kept for the next one: an allocation and a
+  // free of 129 MB took 291 us of an assembly of 384 k tets (2.15 ms, now 1.85).  One call at a time holds it; a call
+  // from another thread meanwhile allocates its own.
+  mutable std::mutex km_lock;
+  mutable bool km_held = false;
+  mutable efm::DevBuf km;
 };

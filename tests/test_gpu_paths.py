@@ -301,3 +301,31 @@ def test_edge_numbering_of_large_buckets(torch_dev, grid):
     np.testing.assert_array_equal(topo.edges.cpu().numpy(), np.array(list(seen)))
     np.testing.assert_array_equal(topo.tet_edges.cpu().numpy(), edges)
     np.testing.assert_array_equal(topo.tet_sign.cpu().numpy(), sign)
+
+
+def test_assembly_scratch_from_two_threads(torch_dev):
+    """Assemblies of one mesh from two threads on two streams share its scratch only one at a
+    time: every result is the single-threaded one, bit for bit."""
+    import threading
+    import torch
+    from edgefem_amd import _capi
+    xyz, tets = _fan_mesh(400, 50)
+    topo = _capi.Topology(np.arange(len(xyz)), tets, np.zeros((0, 3), np.int32))
+    scales = [1.0, 1.5]
+    ref = [[v.clone() for v in _capi.assemble_km(topo, xyz * c, np.full(len(tets), 2.0 + 0j))] for c in scales]
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(20):
+                K, M = _capi.assemble_km(topo, xyz * scales[i], np.full(len(tets), 2.0 + 0j))
+                if not (torch.equal(K, ref[i][0]) and torch.equal(M, ref[i][1])):
+                    bad.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
