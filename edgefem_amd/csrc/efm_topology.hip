@@ -339,49 +339,37 @@ __global__ void k_row_fill(int64_t n, const int32_t *__restrict__ e2t_ptr,
   }
 }
 
-__device__ inline int32_t find_col(const int32_t *__restrict__ col_idx, int32_t lo, int32_t hi,
-                                   int32_t c) {
-  while (lo < hi) {
-    int32_t mid = (lo + hi) >> 1;
-    if (col_idx[mid] < c)
-      lo = mid + 1;
-    else
-      hi = mid;
-  }
-  return lo;
-}
-
 // Contributor lists: for nnz (r, c) every (t, i, j) with tet_edges[t][i] = r and
 // tet_edges[t][j] = c, in ascending t -- the triplet insertion order that
-// setFromTriplets sums in (assemble_maxwell.cpp:185-205).  Each thread owns one row,
-// so the counts and cursors of its nnz are private.
-__global__ void k_contrib(int64_t n, int pass, const int32_t *__restrict__ e2t_ptr,
-                          const int32_t *__restrict__ e2t, const int32_t *__restrict__ tet_edges,
-                          const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col_idx,
-                          int32_t *__restrict__ ccnt, const int32_t *__restrict__ cptr,
-                          int32_t *__restrict__ contrib) {
-  int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= n)
+// setFromTriplets sums in (assemble_maxwell.cpp:185-205).  One thread per nnz looks through the
+// tets of its row (five on average, whose edges the threads of a row share); the first pass
+// counts, the second writes.  58 us per pass for 196 k tets (one thread per row with a search
+// of the row for every local edge: 312).
+__global__ void __launch_bounds__(kBlock)
+    k_contrib(int64_t nnz, int pass, const int32_t *__restrict__ e2t_ptr, const int32_t *__restrict__ e2t,
+              const int32_t *__restrict__ tet_edges, const int32_t *__restrict__ row_idx,
+              const int32_t *__restrict__ col_idx, int32_t *__restrict__ ccnt,
+              const int32_t *__restrict__ cptr, int32_t *__restrict__ contrib) {
+  const int64_t p = (int64_t)blockIdx.x * kBlock + threadIdx.x;
+  if (p >= nnz)
     return;
-  int32_t r0 = row_ptr[e], r1 = row_ptr[e + 1];
-  for (int32_t k = e2t_ptr[e]; k < e2t_ptr[e + 1]; ++k) {
-    int32_t s = e2t[k];
-    int32_t t = s / 6;
-    int32_t i = s - t * 6;
-    for (int j = 0; j < 6; ++j) {
-      int32_t c = tet_edges[(int64_t)t * 6 + j];
-      int32_t pos = find_col(col_idx, r0, r1, c);
-      if (pos >= r1 || col_idx[pos] != c)
-        continue;  // cannot happen: c is in row e by construction
-      if (pass == 0) {
-        ccnt[pos] += 1;
-      } else {
-        int32_t at = cptr[pos] + ccnt[pos];
-        ccnt[pos] += 1;
-        contrib[at] = t * 36 + i * 6 + j;
+  const int32_t r = row_idx[p], c = col_idx[p];
+  int32_t m = 0, at = pass ? cptr[p] : 0;
+  for (int32_t k = e2t_ptr[r]; k < e2t_ptr[r + 1]; ++k) {
+    const int32_t s = e2t[k], t = s / 6;
+    const int2 *te = reinterpret_cast<const int2 *>(tet_edges + (int64_t)t * 6);
+    const int2 a = te[0], b = te[1], d = te[2];
+    const int32_t ed[6] = {a.x, a.y, b.x, b.y, d.x, d.y};
+#pragma unroll
+    for (int j = 0; j < 6; ++j)
+      if (ed[j] == c) {
+        if (pass)
+          contrib[at++] = t * 36 + (s - t * 6) * 6 + j;
+        ++m;
       }
-    }
   }
+  if (!pass)
+    ccnt[p] = m;
 }
 
 } // namespace
@@ -566,10 +554,9 @@ extern "C" int efm_topology_create(int64_t n_nodes, const int64_t *node_ids, int
   ALLOC(ccnt, nnz * 4);
   ALLOC(topo->cptr, (nnz + 1) * 4);
   ALLOC(topo->contrib, T * 36 * 4 + 4);
-  EFM_HIP_CHECK(hipMemsetAsync(ccnt.p, 0, nnz * 4, st));
-  hipLaunchKernelGGL(k_contrib, dim3(grid_for(n, kBlock)), dim3(kBlock), 0, st, n, 0,
+  hipLaunchKernelGGL(k_contrib, dim3(grid_for(nnz, kBlock)), dim3(kBlock), 0, st, nnz, 0,
                      topo->e2t_ptr.as<int32_t>(), topo->e2t.as<int32_t>(),
-                     topo->tet_edges.as<int32_t>(), topo->row_ptr.as<int32_t>(),
+                     topo->tet_edges.as<int32_t>(), topo->row_idx.as<int32_t>(),
                      topo->col_idx.as<int32_t>(), ccnt.as<int32_t>(), nullptr, nullptr);
   EFM_LAUNCH_CHECK();
   int64_t ctot = 0;
@@ -579,10 +566,9 @@ extern "C" int efm_topology_create(int64_t n_nodes, const int64_t *node_ids, int
     set_error("efm_topology_create: contributor count mismatch (internal error)");
     return EFM_ERR_MESH;
   }
-  EFM_HIP_CHECK(hipMemsetAsync(ccnt.p, 0, nnz * 4, st));
-  hipLaunchKernelGGL(k_contrib, dim3(grid_for(n, kBlock)), dim3(kBlock), 0, st, n, 1,
+  hipLaunchKernelGGL(k_contrib, dim3(grid_for(nnz, kBlock)), dim3(kBlock), 0, st, nnz, 1,
                      topo->e2t_ptr.as<int32_t>(), topo->e2t.as<int32_t>(),
-                     topo->tet_edges.as<int32_t>(), topo->row_ptr.as<int32_t>(),
+                     topo->tet_edges.as<int32_t>(), topo->row_idx.as<int32_t>(),
                      topo->col_idx.as<int32_t>(), ccnt.as<int32_t>(), topo->cptr.as<int32_t>(),
                      topo->contrib.as<int32_t>());
   EFM_LAUNCH_CHECK();
