@@ -32,6 +32,7 @@ struct DevBuf {
       return EFM_OK;
     if (hipMalloc(&p, b) != hipSuccess) {
       p = nullptr;
+      (void)hipGetLastError();  // a caller that goes on without the buffer checks its launches
       set_error("hipMalloc of " + std::to_string(b) + " bytes failed");
       return EFM_ERR_NOMEM;
     }

@@ -2416,12 +2416,11 @@ template <int R> struct Dispatch {
         return EFM_OK;
       const int64_t rpb = std::max<int64_t>(kRowsMin, (n + s->ncu - 1) / s->ncu);
       const int nb = (int)((n + rpb - 1) / rpb);
-      int rc;
-      if ((rc = s->ps_lidx.alloc((size_t)s->nnz * 2)) || (rc = s->ps_rloc.alloc((size_t)n * 2)) ||
-          (rc = s->ps_ucol.alloc((size_t)(s->nnz + n) * 4)) || (rc = s->ps_nu.alloc((size_t)nb * 4)) ||
-          (rc = s->ps_part.alloc((size_t)3 * nb * kMaxD * 8)) ||
-          (rc = s->ps_cnt.alloc((size_t)kCounters * kCounterStride * 4 + 128)))
-        return rc;
+      if (s->ps_lidx.alloc((size_t)s->nnz * 2) || s->ps_rloc.alloc((size_t)n * 2) ||
+          s->ps_ucol.alloc((size_t)(s->nnz + n) * 4) || s->ps_nu.alloc((size_t)nb * 4) ||
+          s->ps_part.alloc((size_t)3 * nb * kMaxD * 8) ||
+          s->ps_cnt.alloc((size_t)kCounters * kCounterStride * 4 + 128))
+        return EFM_OK;  // no room: one launch per step
       const size_t lds = (size_t)2 * ((n + 31) / 32) * 4;
       hipLaunchKernelGGL(k_persist_cols, dim3(nb), dim3(kThreads), lds, st, (int)n, (int)rpb, s->row_ptr, s->col,
                          s->ps_lidx.as<uint16_t>(), s->ps_rloc.as<uint16_t>(), s->ps_ucol.as<int32_t>(),
@@ -2458,11 +2457,10 @@ template <int R> struct Dispatch {
   static int persist_solve(efm_solver *s, hipStream_t st, double tol2, int max_it, bool &done) {
     if constexpr (R <= 4) {
       using namespace efm_persist;
-      int rc;
       const bool lr = s->lr_P > 0;
       if (lr && !s->ps_lr_ok) {
-        if ((rc = s->ps_lrport.alloc((size_t)s->n)) || (rc = s->ps_lrw.alloc((size_t)s->n * sizeof(double2))))
-          return rc;
+        if (s->ps_lrport.alloc((size_t)s->n) || s->ps_lrw.alloc((size_t)s->n * sizeof(double2)))
+          return EFM_OK;
         EFM_HIP_CHECK(hipMemsetAsync(s->ps_lrport.p, 0xFF, (size_t)s->n, st));
         const int64_t m = s->lr_P * s->lr_len;
         hipLaunchKernelGGL(k_persist_lr_rows, dim3(grid_for(m, 256)), dim3(256), 0, st, (int)s->n, m, s->lr_len,

@@ -2995,7 +2995,17 @@ extern "C" int efm_sweep_solve(efm_sweep *s, int nsys, const double *h_k0sq, con
   EFM_REQUIRE(s->c_rows == 0 || ((s->c_vals || s->c_nnz == 0) && s->c_nsys == nsys),
               "efm_sweep_solve: correction values missing or set for another number of systems");
   hipStream_t st = (hipStream_t)stream;
-  const bool flat = !h_refine && s->form == 2 && s->spmv_variant < 0 && s->aux_variant < 0 && flat_wins(s->n, nsys);
+  bool flat = !h_refine && s->form == 2 && s->spmv_variant < 0 && s->aux_variant < 0 && flat_wins(s->n, nsys);
+  if (flat && !s->KM.p) {
+    if (s->KM.alloc((size_t)s->nnz * 16) || (s->cplx && s->KMi.alloc((size_t)s->nnz * 16))) {
+      (void)s->KM.alloc(0);  // no room: the padded kernels
+      flat = false;
+    } else {
+      hipLaunchKernelGGL(k_sf_pair, dim3(grid_for(s->nnz, 256)), dim3(256), 0, st, s->nnz, s->K.as<double2>(),
+                         s->M.as<double2>(), s->KM.as<double2>(), s->KMi.as<double2>());
+      EFM_LAUNCH_CHECK();
+    }
+  }
   // the wide kernels' system count is padded to whole wavefronts
   const int Bp = flat ? nsys : ((nsys + kSys - 1) / kSys) * kSys;
   const int P = s->P;
@@ -3027,17 +3037,8 @@ extern "C" int efm_sweep_solve(efm_sweep *s, int nsys, const double *h_k0sq, con
   run.Bp = Bp;
   run.groups = (Bp + kSys - 1) / kSys;
   run.flat = flat;
-  if (flat) {
+  if (flat)
     run.fd = flat_dims(nsys);
-    if (!s->KM.p) {
-      int rc2;
-      if ((rc2 = s->KM.alloc((size_t)s->nnz * 16)) || (s->cplx && (rc2 = s->KMi.alloc((size_t)s->nnz * 16))))
-        return rc2;
-      hipLaunchKernelGGL(k_sf_pair, dim3(grid_for(s->nnz, 256)), dim3(256), 0, st, s->nnz, s->K.as<double2>(),
-                         s->M.as<double2>(), s->KM.as<double2>(), s->KMi.as<double2>());
-      EFM_LAUNCH_CHECK();
-    }
-  }
   run.P = P;
   run.check = h_opts->check_every > 0 ? h_opts->check_every : 16;
   run.tol2 = h_opts->tolerance * h_opts->tolerance;
