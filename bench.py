@@ -794,7 +794,7 @@ def main():
     s_val = 16 if args.mode == "fp64" else 8
     # algorithmic bytes of the chosen SpMV: the fused form reads z and p_old and writes p and
     # q per row and RHS (4 passes); variants 9-11 (p formed in its own pass, tiled, sliced-ELL
-    # or with split values) gather p and write q (2 passes); the sliced-ELL padding slots are
+    # or staged in LDS) gather p and write q (2 passes); the ELL padding slots are
     # not algorithmic bytes, and variant 11's saving (8 B instead of 16 per real value) is
     # not subtracted: the bytes are those of a complex value per entry
     spmv_bytes = nnz * (s_val + 4) + 4 * (n + 1) + R * n * 16 * (2 if variant in (9, 10, 11) else 4)
@@ -836,7 +836,7 @@ def main():
                    "mode": args.mode},
         "roofline": {"bound": "hbm", "achieved": achieved / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK, "traffic": traffic, "traffic_unit": "GB per launch",
-                     "kernel": {9: "k_cocgz_spmv", 10: "k_cocgz_sell", 11: "k_cocgz_spmv (split values)"}.get(variant, "k_cocg_spmv"),
+                     "kernel": {9: "k_cocgz_spmv", 10: "k_cocgz_sell", 11: "k_staged (columns of 512 rows in LDS)"}.get(variant, "k_cocg_spmv"),
                      "bytes_per_launch": spmv_bytes, "avg_launch_ms": avg_ms, "launches": spmv_n,
                      "variant": variant, "autotune_ms": [round(float(t), 4) for t in tune_ms]},
         "cpu_baseline": cpu,
