@@ -642,6 +642,7 @@ def traffic_from_pmc(fetch_csv, write_csv, out_path, variant, commands):
     WRITE_SIZE, KiB per dispatch), each scaled by what the same counter reads for the
     calibration copy (the largest device-to-device copy of the run, of known size)."""
     import csv
+    import re
     import numpy as np
 
     def load(path, counter):
@@ -654,7 +655,7 @@ def traffic_from_pmc(fetch_csv, write_csv, out_path, variant, commands):
             v = float(r["Counter_Value"])
             if name.startswith("__amd_rocclr_copyBuffer"):
                 copy_kib = v if copy_kib is None else max(copy_kib, v)   # the calibration copy is the largest
-            short = name.replace("void ", "").replace("(anonymous namespace)::", "").replace("efm::", "")
+            short = re.sub(r"void |\(anonymous namespace\)::|efm(_staged)?::", "", name)
             per.setdefault(short.split("(")[0], []).append(v)
         return {k: float(np.mean(v)) for k, v in per.items()}, copy_kib
 
@@ -724,7 +725,7 @@ def main():
     if args.traffic_from:
         cmd = ("rocprofv3 --pmc {c} --output-format csv -d pmc_{d} -o {d} -- python -u bench.py --no-cpu "
                "--no-check --steps 1 --warmup 0 --max-it 20 --spmv-variant {v} --calibrate-copy 512")
-        v = args.spmv_variant if args.spmv_variant >= 0 else 9
+        v = args.spmv_variant if args.spmv_variant >= 0 else 11
         traffic_from_pmc(args.traffic_from[0], args.traffic_from[1], os.path.join(ROOT, "profiles", "traffic_c2.json"),
                          v, [cmd.format(c="FETCH_SIZE", d="fetch", v=v), cmd.format(c="WRITE_SIZE", d="write", v=v)])
         return
@@ -809,7 +810,7 @@ def main():
         if tj.get("variant") == variant and args.mode == "fp64":
             for k, v in tj["kernels"].items():
                 # the SpMV of the iteration
-                if k.startswith(("k_cocg_spmv", "k_cocgz_spmv")):
+                if k.startswith(("k_cocg_spmv", "k_cocgz_spmv", "k_staged")):
                     traffic = v["hbm_bytes"] / 1e9
     dS = None
     gold = golden_c2() if not args.small else None
