@@ -3,10 +3,13 @@
 // every cell carries R excitations.  Each (cell, excitation) pair is its own Krylov
 // system with its own alpha, beta, omega, rho and convergence flag.
 //
-// Row tiling: every block owns a contiguous row range inside one cell, so the partial
-// sums of a block belong to one cell and the finalisation of cell c reduces the
-// contiguous block range of c (plus one slot per port term of c).  Nodes of the
-// auxiliary preconditioner are tiled the same way.
+// Row tiling: kRowsPerTile consecutive rows of one cell are a partial sum of its dot
+// products, and the finalisation of cell c reduces the contiguous tile range of c (plus one
+// slot per port term of c).  The tiles, and the order of the additions in each, depend on the
+// cell alone: its iterates do not change with the cells that share the batch (BiCGSTAB on
+// these systems ends elsewhere below the tolerance when a sum is regrouped).  How many blocks
+// work on a tile is another matter, see split_tiles.  Nodes of the auxiliary preconditioner
+// are tiled the same way, without sums across a tile.
 //
 // Iteration (van der Vorst 1992, right-preconditioned with P = D^{-1} + G Dn^{-1} G^T,
 // the periodic auxiliary preconditioner with a complex incidence; the port loading
@@ -28,13 +31,15 @@ using namespace efm;
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kRowsPerTile = 1024;  // at most
+constexpr int kRowsPerTile = 1024;
 constexpr int kLanes = 8;  // SpMV lanes per row
 constexpr int kMaxR = 2;
-constexpr int kMinTiles = 1600;  // row tiles wanted of a batch that can have them (subs_per_tile)
+constexpr int kMinTiles = 1600;  // blocks wanted of a batch that can have them (subs_per_block)
+constexpr int kXThreads = 1024;  // of k_cells_x where few tiles would leave most CUs idle
 // Nodes per block of the nodal kernel: two rounds of 32 nodes.  A tile of 1,024 nodes is 32
 // serial rounds of dependent loads on a grid of one block per 1,024 nodes: 54.0 us per
-// launch on 12 cells (60 blocks) against 6.7 us with 64 nodes.
+// launch on 12 cells (60 blocks) against 6.7 us with 64 nodes; 512 cells, all active: 702
+// against 524 us (256 nodes: 547).
 constexpr int kNodesPerTile = 64;
 
 struct CellSys {
@@ -63,7 +68,14 @@ struct Tile {
 
 __device__ inline double2 bil(double2 a, double2 b) { return cmul(a, b); }
 
-// block sum of V complex values; result in lds[0..V) for all threads
+// |a|^2 with its roundings written out, for sums that two kernels form: the compiler contracts
+// a.x a.x + a.y a.y either way round.
+template <bool Y_OUTER> __device__ inline double norm2(double2 a) {
+  return Y_OUTER ? fma(a.y, a.y, a.x * a.x) : fma(a.x, a.x, a.y * a.y);
+}
+
+// block sum of V complex values over the first kBlock threads; result in lds[0..V) for all
+// threads (lds: V per wavefront of the block)
 template <int V>
 __device__ inline void bsum(double2 (&v)[V], double2 *lds) {
 #pragma unroll
@@ -496,11 +508,12 @@ __global__ void __launch_bounds__(kBlock)
 // walks its sub-tiles sdesc[soff[t] .. soff[t+1]) of at most kSubNnz entries and kSubRows
 // rows; each thread streams 4 entries of a sub-tile (branch-free loads, the next sub-tile's
 // in flight during the gathers), the products go to LDS and kSubRL lanes per row sum them.
+// DOT false: tiles of fewer sub-tiles, without the partials (k_cells_dot makes them).
 constexpr int kSubNnz = 1024;
 constexpr int kSubRL = 4;
 constexpr int kSubRows = kBlock / kSubRL;
 
-template <int R, int MODE>
+template <int R, int MODE, bool DOT>
 __global__ void __launch_bounds__(kBlock)
     k_cells_spmv_t(const Tile *__restrict__ tiles, const int32_t *__restrict__ soff, const int4 *__restrict__ sdesc,
                    const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col,
@@ -585,18 +598,74 @@ __global__ void __launch_bounds__(kBlock)
           continue;
         const int64_t k = (int64_t)row * R + s;
         out[k] = acc[s];
+        if (!DOT)
+          continue;
         const double2 o = other[k];
         if (MODE == 0) {
           d[s] = cfma(cconj(o), acc[s], d[s]);
         } else {
           d[s] = cfma(cconj(acc[s]), o, d[s]);
-          d[R + s].x += cabs2(acc[s]);
+          d[R + s].x += norm2<R == 1>(acc[s]);
         }
       }
     }
     __syncthreads();  // prod is reused by the next sub-tile
     cur = nxt;
   }
+  if (DOT)
+    put_partials<V>(d, lds, partial, blockIdx.x);
+}
+
+// The partials of k_cells_spmv_t for a tile whose rows several blocks have multiplied: the
+// tile's rows into LDS, then the same threads add the same rows in the same order.
+template <int R, int MODE>
+__global__ void __launch_bounds__(kBlock)
+    k_cells_dot(const Tile *__restrict__ tiles, const int32_t *__restrict__ soff, const int4 *__restrict__ sdesc,
+                const double2 *__restrict__ out, const double2 *__restrict__ other, double2 *__restrict__ partial,
+                const CellSys *__restrict__ st) {
+  constexpr int V = MODE == 0 ? R : 2 * R;
+  __shared__ double2 lo[R * kRowsPerTile], lt[R * kRowsPerTile];
+  __shared__ double2 lds[(kBlock / 64) * 2 * kMaxR];
+  const Tile t = tiles[blockIdx.x];
+  if (!cell_active<R>(st, t.cell))
+    return;
+  bool act[R];
+#pragma unroll
+  for (int s = 0; s < R; ++s)
+    act[s] = st[(int64_t)t.cell * R + s].active != 0;
+  const int m = (int)(t.r1 - t.r0) * R;  // <= R * kRowsPerTile
+#pragma unroll
+  for (int q = 0; q < R * kRowsPerTile / kBlock; ++q) {
+    const int i = threadIdx.x + q * kBlock;
+    const int64_t k = t.r0 * R + (i < m ? i : 0);
+    lo[i] = out[k];
+    lt[i] = other[k];
+  }
+  double2 d[V];
+#pragma unroll
+  for (int s = 0; s < V; ++s)
+    d[s] = make_double2(0, 0);
+  __syncthreads();
+  const int g = threadIdx.x / kSubRL;
+  if (threadIdx.x % kSubRL == 0)
+    for (int j = soff[blockIdx.x]; j < soff[blockIdx.x + 1]; ++j) {
+      const int4 dsc = sdesc[j];
+      if (dsc.x + g >= dsc.y)
+        continue;
+      const int i = (int)(dsc.x + g - t.r0) * R;
+#pragma unroll
+      for (int s = 0; s < R; ++s) {
+        if (!act[s])
+          continue;
+        const double2 a = lo[i + s], o = lt[i + s];
+        if (MODE == 0) {
+          d[s] = cfma(cconj(o), a, d[s]);
+        } else {
+          d[s] = cfma(cconj(a), o, d[s]);
+          d[R + s].x += norm2<R == 1>(a);
+        }
+      }
+    }
   put_partials<V>(d, lds, partial, blockIdx.x);
 }
 
@@ -696,13 +765,18 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
-// x += alpha y + omega zz; r = s - omega t; partials r0^H r, |r|^2
-template <int R>
-__global__ void __launch_bounds__(kBlock)
+// x += alpha y + omega zz; r = s - omega t; partials r0^H r, |r|^2.  NT threads; with more than
+// kBlock the elements' terms go through LDS, and the first kBlock threads add the ones that
+// they would have had alone, in the same order.
+template <int R, int NT>
+__global__ void __launch_bounds__(NT)
     k_cells_x(const Tile *__restrict__ tiles, const double2 *__restrict__ y, const double2 *__restrict__ zz,
               const double2 *__restrict__ tvec, const double2 *__restrict__ r0, double2 *__restrict__ x,
               double2 *__restrict__ r, double2 *__restrict__ partial, const CellSys *__restrict__ st) {
-  __shared__ double2 lds[(kBlock / 64) * 2 * kMaxR];
+  constexpr bool kStaged = NT > kBlock;
+  __shared__ double2 lds[(NT / 64) * 2 * kMaxR];
+  __shared__ double2 ldr[kStaged ? R * kRowsPerTile : 1];
+  __shared__ double lrr[kStaged ? R * kRowsPerTile : 1];
   const Tile t = tiles[blockIdx.x];
   if (!cell_active<R>(st, t.cell))  // the finalisation ignores the partials of inactive systems
     return;
@@ -719,7 +793,7 @@ __global__ void __launch_bounds__(kBlock)
 #pragma unroll
   for (int s = 0; s < 2 * R; ++s)
     d[s] = make_double2(0, 0);
-  for (int64_t k = t.r0 * R + threadIdx.x; k < t.r1 * R; k += kBlock) {
+  for (int64_t k = t.r0 * R + threadIdx.x; k < t.r1 * R; k += NT) {
     const int sys = (int)(k % R);
     bool a = false;
     double2 al = make_double2(0, 0), om = make_double2(0, 0);
@@ -730,19 +804,41 @@ __global__ void __launch_bounds__(kBlock)
         al = alpha[s];
         om = omega[s];
       }
-    if (!a)
+    if (!a) {
+      if (kStaged) {
+        ldr[k - t.r0 * R] = make_double2(0, 0);
+        lrr[k - t.r0 * R] = 0.0;
+      }
       continue;
+    }
     x[k] = cadd(x[k], cadd(bil(al, y[k]), bil(om, zz[k])));
     const double2 rv = csub(r[k], bil(om, tvec[k]));
     r[k] = rv;
     const double2 dr = cfma(cconj(r0[k]), rv, make_double2(0, 0));
-    const double rr = cabs2(rv);
+    const double rr = norm2<false>(rv);
+    if (kStaged) {
+      ldr[k - t.r0 * R] = dr;
+      lrr[k - t.r0 * R] = rr;
+      continue;
+    }
 #pragma unroll
     for (int s = 0; s < R; ++s)
       if (s == sys) {
         d[s] = cadd(d[s], dr);
         d[R + s].x += rr;
       }
+  }
+  if (kStaged) {
+    __syncthreads();
+    const int m = (int)(t.r1 - t.r0) * R, sys = threadIdx.x % R;  // kBlock and the first element are multiples of R
+    if (threadIdx.x < kBlock)
+      for (int k = threadIdx.x; k < m; k += kBlock)
+#pragma unroll
+        for (int s = 0; s < R; ++s)
+          if (s == sys) {
+            d[s] = cadd(d[s], ldr[k]);
+            d[R + s].x += lrr[k];
+          }
   }
   put_partials<2 * R>(d, lds, partial, blockIdx.x);
 }
@@ -897,6 +993,8 @@ struct efm_cells {
   efm::DevBuf poff, pidx, pw, pcoef, pcell;
   efm::DevBuf x, r, r0, p, v, y, zz, t, partial, state, flags;
   efm::DevBuf soff, sdesc;  // entry sub-tiles of the row tiles (nsub = 0: not built)
+  efm::DevBuf btiles, bsoff;  // rows and sub-tiles of a block where several work on a tile
+  int64_t nbtiles = 0;        // 0: a block per tile
   int64_t nsub = 0;
   int spmv = 0;  // 1: k_cells_spmv_t on the sub-tiles, 0: row-parallel k_cells_spmv
 };
@@ -927,42 +1025,47 @@ std::vector<Tile> make_tiles(const int64_t *off, int64_t ncells, int64_t per_til
   return t;
 }
 
-// Sub-tiles per row tile (one block each in every row kernel).  A tile is one block's
-// serial walk, so few tiles leave most CUs idle and the last round of blocks nearly empty;
-// many tiles cost the finalisation more slots and lose the overlap of one sub-tile's loads
-// with the previous one's gathers.  Measured on 12 cells, 0.4 M rows (whole batch): 16
-// sub-tiles 317 ms, 7 (one round of resident blocks) 275, 4: 211, 2: 217, 1: 200 (4 and
-// below are alike up to the iteration counts); 512 cells, 27 M rows, run with 16.
-int subs_per_tile(int64_t n) {
+// Entry sub-tiles of every row tile: at most kSubNnz entries and kSubRows rows of one tile.
+// False when a row holds more than kSubNnz entries.
+bool make_sub_tiles(const std::vector<Tile> &tiles, const int32_t *rp, std::vector<int4> &sd,
+                    std::vector<int32_t> &so) {
+  for (const Tile &t : tiles) {
+    so.push_back((int32_t)sd.size());
+    for (int64_t r = t.r0; r < t.r1;) {
+      int64_t r1 = r;
+      while (r1 < t.r1 && r1 - r < kSubRows && rp[r1 + 1] - rp[r] <= kSubNnz)
+        ++r1;
+      if (r1 == r)
+        return false;
+      sd.push_back(make_int4((int32_t)r, (int32_t)r1, rp[r], rp[r1]));
+      r = r1;
+    }
+  }
+  so.push_back((int32_t)sd.size());
+  return true;
+}
+
+// Sub-tiles per block of the row kernels.  A block walks its sub-tiles one after another, so a
+// batch of few tiles with a block each leaves most CUs idle and the last round of blocks nearly
+// empty; many blocks lose the overlap of one sub-tile's loads with the previous one's
+// gathers, and the products' dot products then take a kernel of their own (k_cells_dot), which
+// reads both vectors again.  With half a tile per block or more that costs what it gives, and a
+// block takes a tile.  us per iteration, a block per tile against this: 1 cell (53 k rows) 159,
+// 93; 4: 173, 150; 8: 230, 210; 12: 284, 263; 16: 386, 379; 24 (1.3 M rows, if split) 581, 640.
+int subs_per_block(int64_t n) {
   const int64_t subs = n / kSubRows;
   return (int)std::max<int64_t>(1, std::min<int64_t>(kRowsPerTile / kSubRows, subs / kMinTiles));
 }
 
-// Row tiles of up to `subs` whole entry sub-tiles (sub-tile: at most kSubNnz entries and
-// kSubRows rows of one cell).  False when a row holds more than kSubNnz entries.
-bool make_row_tiles(const int64_t *off, int64_t ncells, const int32_t *rp, int subs, std::vector<Tile> &tiles,
-                    std::vector<int32_t> &first, std::vector<int4> &sd, std::vector<int32_t> &so) {
-  first.assign(ncells + 1, 0);
-  for (int64_t c = 0; c < ncells; ++c) {
-    first[c] = (int32_t)tiles.size();
-    for (int64_t r = off[c]; r < off[c + 1];) {
-      const int64_t r0 = r;
-      so.push_back((int32_t)sd.size());
-      for (int k = 0; k < subs && r < off[c + 1]; ++k) {
-        int64_t r1 = r;
-        while (r1 < off[c + 1] && r1 - r < kSubRows && rp[r1 + 1] - rp[r] <= kSubNnz)
-          ++r1;
-        if (r1 == r)
-          return false;
-        sd.push_back(make_int4((int32_t)r, (int32_t)r1, rp[r], rp[r1]));
-        r = r1;
-      }
-      tiles.push_back(Tile{(int32_t)c, 0, r0, r});
+// Blocks of `subs` sub-tiles each, none across two row tiles.
+void split_tiles(const std::vector<Tile> &tiles, const std::vector<int4> &sd, const std::vector<int32_t> &so, int subs,
+                 std::vector<Tile> &bt, std::vector<int32_t> &bso) {
+  for (size_t t = 0; t < tiles.size(); ++t)
+    for (int32_t j = so[t]; j < so[t + 1]; j += subs) {
+      bso.push_back(j);
+      bt.push_back(Tile{tiles[t].cell, 0, sd[j].x, sd[std::min(j + subs, so[t + 1]) - 1].y});
     }
-  }
-  first[ncells] = (int32_t)tiles.size();
-  so.push_back((int32_t)sd.size());
-  return true;
+  bso.push_back((int32_t)sd.size());
 }
 } // namespace
 
@@ -1020,23 +1123,26 @@ extern "C" int efm_cells_create(int64_t ncells, const int64_t *h_row_off, const 
     EFM_HIP_CHECK(hipStreamSynchronize(st));
     EFM_REQUIRE(last == nnz, "efm_cells_create: row_ptr[n] != nnz");
   }
-  // row tiles, and the entry sub-tiles of each for the SpMV
-  std::vector<int32_t> first, so;
-  std::vector<Tile> tiles;
+  // row tiles, the entry sub-tiles of each for the SpMV, and the blocks' shares of them
+  std::vector<int32_t> first, so, bso;
+  std::vector<Tile> tiles = make_tiles(h_row_off, ncells, kRowsPerTile, &first), bt;
   std::vector<int4> sd;
   {
     std::vector<int32_t> hrp(n + 1);
     EFM_HIP_CHECK(hipMemcpy(hrp.data(), s->row_ptr.p, (n + 1) * sizeof(int32_t), hipMemcpyDeviceToHost));
-    if (!make_row_tiles(h_row_off, ncells, hrp.data(), subs_per_tile(n), tiles, first, sd, so)) {
-      // a row longer than a sub-tile: keep the row-parallel kernel
-      tiles = make_tiles(h_row_off, ncells, kRowsPerTile, &first);
-      sd.clear();
-    }
-    if (!sd.empty()) {
+    // without sub-tiles (a row longer than one): the row-parallel kernel
+    if (make_sub_tiles(tiles, hrp.data(), sd, so) && !sd.empty()) {
       if ((rc = upload(s->sdesc, sd.data(), sd.size(), st)) || (rc = upload(s->soff, so.data(), so.size(), st)))
         return rc;
       s->nsub = (int64_t)sd.size();
       s->spmv = 1;
+      const int subs = subs_per_block(n);
+      if (2 * subs < kRowsPerTile / kSubRows) {
+        split_tiles(tiles, sd, so, subs, bt, bso);
+        if ((rc = upload(s->btiles, bt.data(), bt.size(), st)) || (rc = upload(s->bsoff, bso.data(), bso.size(), st)))
+          return rc;
+        s->nbtiles = (int64_t)bt.size();
+      }
     }
   }
   std::vector<Tile> ntl = make_tiles(h_node_off, ncells, kNodesPerTile, nullptr);
@@ -1160,6 +1266,9 @@ template <int R> int cells_solve(efm_cells *s, const double2 *B, double2 *X, con
   CellSys *S = s->state.as<CellSys>();
   double2 *part = s->partial.as<double2>();
   const int nt = (int)s->ntiles, nnt = (int)s->nntiles, nc = (int)s->ncells;
+  const bool split = s->nbtiles > 0;
+  const Tile *BT = split ? s->btiles.as<Tile>() : T;  // rows of a block of the kernels without sums
+  const int nbt = split ? (int)s->nbtiles : nt;
   const double tol2 = o->tolerance * o->tolerance;
   const int max_it = o->max_iterations;
   const int check = o->check_every > 0 ? o->check_every : 32;
@@ -1180,9 +1289,29 @@ template <int R> int cells_solve(efm_cells *s, const double2 *B, double2 *X, con
                          s->ynode.as<double2>(), S);
       EFM_LAUNCH_CHECK();
     }
-    hipLaunchKernelGGL((k_cells_aux_edge<R>), dim3(nt), dim3(kBlock), 0, st, T, s->en2.as<int2>(),
+    hipLaunchKernelGGL((k_cells_aux_edge<R>), dim3(nbt), dim3(kBlock), 0, st, BT, s->en2.as<int2>(),
                        s->ga.as<double2>(), s->gb.as<double2>(), s->dinv.as<double2>(), s->ynode.as<double2>(), in,
                        outv, S);
+    EFM_LAUNCH_CHECK();
+    return EFM_OK;
+  };
+  auto spmv = [&](auto mode_tag, const double2 *in, double2 *outv, const double2 *other) -> int {
+    constexpr int MODE = decltype(mode_tag)::value;
+    const int32_t *rp = s->row_ptr.as<int32_t>(), *ci = s->col.as<int32_t>(), *so = s->soff.as<int32_t>();
+    const int4 *sd = s->sdesc.as<int4>();
+    const double2 *va = s->val.as<double2>();
+    if (s->spmv == 1 && split) {
+      hipLaunchKernelGGL((k_cells_spmv_t<R, MODE, false>), dim3(nbt), dim3(kBlock), 0, st, BT, s->bsoff.as<int32_t>(),
+                         sd, rp, ci, va, in, outv, other, part, S);
+      EFM_LAUNCH_CHECK();
+      hipLaunchKernelGGL((k_cells_dot<R, MODE>), dim3(nt), dim3(kBlock), 0, st, T, so, sd, outv, other, part, S);
+    } else if (s->spmv == 1) {
+      hipLaunchKernelGGL((k_cells_spmv_t<R, MODE, true>), dim3(nt), dim3(kBlock), 0, st, T, so, sd, rp, ci, va, in,
+                         outv, other, part, S);
+    } else {
+      hipLaunchKernelGGL((k_cells_spmv<R, MODE>), dim3(nt), dim3(kBlock), 0, st, T, rp, ci, va, in, outv, other, part,
+                         S);
+    }
     EFM_LAUNCH_CHECK();
     return EFM_OK;
   };
@@ -1225,35 +1354,22 @@ template <int R> int cells_solve(efm_cells *s, const double2 *B, double2 *X, con
         if ((rc = fin(std::integral_constant<int, kRho0>{})))
           return rc;
       }
-      hipLaunchKernelGGL((k_cells_p<R>), dim3(nt), dim3(kBlock), 0, st, T, r, v, p, r0, S);
+      hipLaunchKernelGGL((k_cells_p<R>), dim3(nbt), dim3(kBlock), 0, st, BT, r, v, p, r0, S);
       EFM_LAUNCH_CHECK();
       if ((rc = precond(p, y)))
         return rc;
-      if (s->spmv == 1)
-        hipLaunchKernelGGL((k_cells_spmv_t<R, 0>), dim3(nt), dim3(kBlock), 0, st, T, s->soff.as<int32_t>(),
-                           s->sdesc.as<int4>(), s->row_ptr.as<int32_t>(), s->col.as<int32_t>(),
-                           s->val.as<double2>(), y, v, r0, part, S);
-      else
-        hipLaunchKernelGGL((k_cells_spmv<R, 0>), dim3(nt), dim3(kBlock), 0, st, T, s->row_ptr.as<int32_t>(),
-                           s->col.as<int32_t>(), s->val.as<double2>(), y, v, r0, part, S);
-      EFM_LAUNCH_CHECK();
-      if ((rc = ports(I0{}, y, v, r0)) || (rc = fin(std::integral_constant<int, kAlpha>{})))
+      if ((rc = spmv(I0{}, y, v, r0)) || (rc = ports(I0{}, y, v, r0)) || (rc = fin(std::integral_constant<int, kAlpha>{})))
         return rc;
-      hipLaunchKernelGGL((k_cells_s<R>), dim3(nt), dim3(kBlock), 0, st, T, v, r, S);
+      hipLaunchKernelGGL((k_cells_s<R>), dim3(nbt), dim3(kBlock), 0, st, BT, v, r, S);
       EFM_LAUNCH_CHECK();
       if ((rc = precond(r, zz)))
         return rc;
-      if (s->spmv == 1)
-        hipLaunchKernelGGL((k_cells_spmv_t<R, 1>), dim3(nt), dim3(kBlock), 0, st, T, s->soff.as<int32_t>(),
-                           s->sdesc.as<int4>(), s->row_ptr.as<int32_t>(), s->col.as<int32_t>(),
-                           s->val.as<double2>(), zz, t, r, part, S);
-      else
-        hipLaunchKernelGGL((k_cells_spmv<R, 1>), dim3(nt), dim3(kBlock), 0, st, T, s->row_ptr.as<int32_t>(),
-                           s->col.as<int32_t>(), s->val.as<double2>(), zz, t, r, part, S);
-      EFM_LAUNCH_CHECK();
-      if ((rc = ports(I1{}, zz, t, r)) || (rc = fin(std::integral_constant<int, kOmega>{})))
+      if ((rc = spmv(I1{}, zz, t, r)) || (rc = ports(I1{}, zz, t, r)) || (rc = fin(std::integral_constant<int, kOmega>{})))
         return rc;
-      hipLaunchKernelGGL((k_cells_x<R>), dim3(nt), dim3(kBlock), 0, st, T, y, zz, t, r0, x, r, part, S);
+      if (split)
+        hipLaunchKernelGGL((k_cells_x<R, kXThreads>), dim3(nt), dim3(kXThreads), 0, st, T, y, zz, t, r0, x, r, part, S);
+      else
+        hipLaunchKernelGGL((k_cells_x<R, kBlock>), dim3(nt), dim3(kBlock), 0, st, T, y, zz, t, r0, x, r, part, S);
       EFM_LAUNCH_CHECK();
       if ((rc = fin(std::integral_constant<int, kX>{})))
         return rc;

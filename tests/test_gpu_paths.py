@@ -42,6 +42,43 @@ def test_cell_batch_tile_edges_vs_dense_solve(torch_dev, sizes, nrhs):
     batch.close()
 
 
+def _with_filler(inputs, B, rows):
+    """The batch with one cell more: a diagonal of `rows` rows without nodes, solved at once."""
+    ro, rp, col, val, no, en, ec, nrhs, po, pi, pw, pc = inputs
+    n, k = int(ro[-1]), np.arange(rows)
+    out = (np.append(ro, n + rows), np.concatenate([rp, rp[-1] + 1 + k]).astype(np.int32),
+           np.concatenate([col, n + k]).astype(np.int32), np.concatenate([val, np.full(rows, 2.0 + 0.5j)]),
+           np.append(no, no[-1]), np.concatenate([en.reshape(-1), np.full(2 * rows, -1)]).astype(np.int32),
+           np.concatenate([ec.reshape(-1), np.zeros(2 * rows)]), nrhs, np.concatenate([po, np.full(nrhs, po[-1])]), pi, pw,
+           np.concatenate([pc, np.zeros(nrhs)]))
+    return out, np.concatenate([B, np.ones((rows, nrhs))])
+
+
+@pytest.mark.parametrize("nrhs", [1, 2])
+def test_cell_result_does_not_depend_on_the_batch(torch_dev, nrhs):
+    """Cells of one to three row tiles alone and beside a cell of 250 k and of 1.7 M rows (one, two
+    and all sub-tiles of a tile per block): the sums of a cell are the same in every batch, so its
+    solution, iterations and residual are, bit for bit."""
+    from edgefem_amd import _capi
+    from test_gpu_parity import _ragged_cells
+    inputs, B, Xref = _ragged_cells([700, 1024, 1500, 2100], nrhs=nrhs, seed=5)
+    n, ref = B.shape[0], None
+    for rows in (0, 250_000, 1_700_000):
+        cells, rhs = _with_filler(inputs, B, rows) if rows else (inputs, B)
+        batch = _capi.CellBatch(*cells)
+        X, iters, resid = batch.solve(torch_dev.from_numpy(rhs).cuda(), tol=1e-12)
+        X = X.cpu().numpy().reshape(-1, nrhs)
+        batch.close()
+        print(f"nrhs {nrhs}, {rows} rows beside: iterations {iters[:4].ravel()}", flush=True)
+        assert resid.max() <= 1e-12
+        if rows:
+            np.testing.assert_array_equal(X[n:], rhs[n:] / (2.0 + 0.5j))
+        got = X[:n], iters[:4], resid[:4]
+        ref = ref or got
+        for a, b in zip(got, ref):
+            np.testing.assert_array_equal(a, b)
+
+
 def _local_system(n, nrhs, seed, long_rows=()):
     """A complex-symmetric, diagonally dominant matrix (condition number below 10) whose
     rows couple to neighbours at most 40 away, 5 to 15 entries each and about 40 in
