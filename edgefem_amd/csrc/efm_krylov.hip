@@ -1799,7 +1799,9 @@ struct efm_solver {
   int64_t st_pairs = 0;
   bool st_vals_ok = false;
   int grid_rows[3] = {8, 8, 8};
-  int spmv_variant = -1;  // -1: choose by timing at the first solve
+  int spmv_variant = -1;  // set by the caller, or by the tuner (-1: not yet)
+  bool tuned = false;     // by the tuner: a solve that the one kernel covers does not use it
+  bool last_persist = false;
   double tune_ms[kNumSpmvVariants] = {0};
   // auxiliary gradient preconditioner (non-owning mesh arrays)
   bool aux = false;
@@ -2273,6 +2275,7 @@ template <int R> struct Dispatch {
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     s->spmv_variant = best;
+    s->tuned = true;
     return EFM_OK;
   }
 
@@ -2968,12 +2971,14 @@ extern "C" int efm_solver_set_spmv_variant(efm_solver *s, int variant) {
   EFM_REQUIRE(variant != kSplitForm || s->vtype == EFM_C128,
               "efm_solver_set_spmv_variant: variant 11 needs complex-double matrix values");
   s->spmv_variant = variant;
+  s->tuned = false;
+  s->last_persist = false;
   return EFM_OK;
 }
 
 extern "C" int efm_solver_get_spmv_variant(const efm_solver *s, int *h_variant, double *h_tune_ms) {
   EFM_REQUIRE(s && h_variant, "efm_solver_get_spmv_variant: NULL argument");
-  *h_variant = s->spmv_variant;
+  *h_variant = s->last_persist ? -1 : s->spmv_variant;
   if (h_tune_ms)
     for (int v = 0; v < kNumSpmvVariants; ++v)
       h_tune_ms[v] = s->tune_ms[v];
@@ -3038,7 +3043,7 @@ extern "C" int efm_solver_solve(efm_solver *s, const double *B, double *X,
   // Systems whose matrix fits in the register files run in the persistent kernel: 780 rows 21.6
   // (five launches) against 13.3 us per iteration, 31 k 29 against 18.4, 103 k 43 against 33.0.
   bool persist = false;
-  if (cocg && !s->profile && s->spmv_variant < 0) {
+  if (cocg && !s->profile && (s->spmv_variant < 0 || s->tuned)) {
     rc = with_rhs(s->R, [&](auto RC) -> int {
       constexpr int R = decltype(RC)::value;
       if (!Dispatch<R>::persist_covers(s))
@@ -3064,6 +3069,7 @@ extern "C" int efm_solver_solve(efm_solver *s, const double *B, double *X,
         return rc;
     }
   }
+  s->last_persist = persist;
   if (cocg && !persist && s->spmv_variant < 0) {
     rc = with_rhs(s->R, [&](auto RC) -> int {
       constexpr int R = decltype(RC)::value;
@@ -3108,7 +3114,8 @@ extern "C" int efm_solver_solve(efm_solver *s, const double *B, double *X,
       }
     }
   }
-  if (cocg && (s->spmv_variant == kZForm || s->spmv_variant == kSellForm || s->spmv_variant == kSplitForm)) {
+  if (cocg && !persist &&
+      (s->spmv_variant == kZForm || s->spmv_variant == kSellForm || s->spmv_variant == kSplitForm)) {
     // the last iteration's x updates (the p pass makes them one iteration late)
     rc = with_rhs(s->R, [&](auto RC) -> int {
       constexpr int R = decltype(RC)::value;

@@ -196,9 +196,10 @@ int efm_solver_solve(efm_solver *s, const double *B, double *X, const efm_solve_
  * sides where the columns of every 512 rows fit, those columns staged in LDS.  By
  * default (-1) complex-double COCG solves of up to 512 rows per CU (256 with three or four
  * right-hand sides; at most four low-rank terms times right-hand sides) run in one
- * persistent kernel that keeps the matrix in registers and LDS (get reports -1); for
- * others the first solve times variants 0-11 on the installed matrix and keeps the
- * fastest; a fixed variant makes results reproducible bit for bit across runs.
+ * persistent kernel that keeps the matrix in registers and LDS (get reports -1); the first
+ * other solve (a profiled one, too) times variants 0-11 on the installed matrix and keeps
+ * the fastest for solves of its kind; a fixed variant makes results reproducible bit for
+ * bit across runs.
  * h_tune_ms (12 entries, may be NULL) receives the
  * measured average ms per launch (-1 = not available).  No reference counterpart. */
 int efm_solver_set_spmv_variant(efm_solver *s, int variant);

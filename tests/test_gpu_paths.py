@@ -197,6 +197,45 @@ def test_systems_past_the_persistent_kernel(torch_dev, n, nrhs, dtype, terms):
     assert np.linalg.norm(r) <= (2e-10 if dtype == "complex128" else 1e-6) * np.linalg.norm(B)
 
 
+def test_tuned_solver_keeps_the_persistent_kernel(torch_dev):
+    """A profiled solve and one with too many low-rank terms time the variants; what they chose does
+    not change a later solve that the one kernel covers: the same bits as a fresh solver's."""
+    import torch
+    from edgefem_amd import _capi
+    n = 600
+    A, en, B = _local_system(n, 2, 4)
+    rows, w, c = _lowrank_terms(n, 3, np.random.default_rng(2))
+    b = torch.from_numpy(B).cuda()
+
+    def solver():
+        s = _capi.KrylovSolver(A.indptr, A.indices, nrhs=2)
+        s.set_gradient(_Nodes(en))
+        s.set_matrix(A.data)
+        return s
+
+    ref, _ = solver().solve(b, tol=1e-12)
+    s = solver()
+    s.profile(True)
+    s.solve(b, tol=1e-12)
+    assert s.spmv_variant()[0] >= 0
+    s.profile(False)
+    X, info = s.solve(b, tol=1e-12)
+    assert s.spmv_variant()[0] == -1 and info["converged"] and torch.equal(X, ref)
+    s = solver()
+    s.set_lowrank(rows.reshape(-1), w.reshape(-1), c)   # 3 terms and 2 right-hand sides: not covered
+    s.set_matrix(A.data)
+    s.solve(b, tol=1e-12)
+    assert s.spmv_variant()[0] >= 0
+    s.set_lowrank(rows[:0].reshape(-1), w[:0].reshape(-1), c[:0])
+    s.set_matrix(A.data)
+    X, info = s.solve(b, tol=1e-12)
+    assert s.spmv_variant()[0] == -1 and info["converged"] and torch.equal(X, ref)
+    s.set_spmv_variant(0)
+    assert s.spmv_variant()[0] == 0
+    s.solve(b, tol=1e-12)
+    assert s.spmv_variant()[0] == 0
+
+
 def _fan_mesh(levels, ring):
     """Tetrahedra around an axis: axis edges with 3 ring + 1 entries in their rows, axis nodes
     of degree 2 ring + 2."""
