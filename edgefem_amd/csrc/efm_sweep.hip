@@ -2094,6 +2094,9 @@ struct efm_sweep {
   // nodal kernel: 0 = one block slice per system group, 1 = pipelined, XCD-local node
   // walk (groups in turn); -1 = chosen on the first solve (in-place timing, as for the SpMV)
   int aux_variant = -1;
+  // what the caller set: with both -1 a narrow batch is packed, whatever a wide one before it chose
+  int spmv_pinned = -1, aux_pinned = -1;
+  bool last_flat = false;
   int gx_aux = 8;
   int cplx = 3;  // bit 1: K complex, bit 2: M complex (selects the SpMV instantiation)
   // iteration: 0 = standard COCG (p in its own pass, two reductions), 1 = Chronopoulos-Gear,
@@ -2303,8 +2306,9 @@ extern "C" int efm_sweep_set_variants(efm_sweep *s, int spmv, int aux) {
               "efm_sweep_set_variants: SpMV variant must be -1..2, nodal variant -1..1");
   EFM_REQUIRE(spmv != 2 || s->tiled_ok,
               "efm_sweep_set_variants: the LDS-tiled SpMV (2) does not fit this matrix's row tiles");
-  s->spmv_variant = spmv;
-  s->aux_variant = aux;
+  s->spmv_variant = s->spmv_pinned = spmv;
+  s->aux_variant = s->aux_pinned = aux;
+  s->last_flat = false;
   return EFM_OK;
 }
 
@@ -2417,8 +2421,8 @@ extern "C" int efm_sweep_set_iteration(efm_sweep *s, int form) {
 
 extern "C" int efm_sweep_get_variants(const efm_sweep *s, int *h_spmv, int *h_aux, double *h_tune_ms) {
   EFM_REQUIRE(s && h_spmv && h_aux, "efm_sweep_get_variants: NULL argument");
-  *h_spmv = s->spmv_variant;
-  *h_aux = s->aux_variant;
+  *h_spmv = s->last_flat ? -1 : s->spmv_variant;
+  *h_aux = s->last_flat ? -1 : s->aux_variant;
   if (h_tune_ms)
     for (int v = 0; v < 5; ++v)
       h_tune_ms[v] = s->tune_ms[v];
@@ -2995,7 +2999,7 @@ extern "C" int efm_sweep_solve(efm_sweep *s, int nsys, const double *h_k0sq, con
   EFM_REQUIRE(s->c_rows == 0 || ((s->c_vals || s->c_nnz == 0) && s->c_nsys == nsys),
               "efm_sweep_solve: correction values missing or set for another number of systems");
   hipStream_t st = (hipStream_t)stream;
-  bool flat = !h_refine && s->form == 2 && s->spmv_variant < 0 && s->aux_variant < 0 && flat_wins(s->n, nsys);
+  bool flat = !h_refine && s->form == 2 && s->spmv_pinned < 0 && s->aux_pinned < 0 && flat_wins(s->n, nsys);
   if (flat && !s->KM.p) {
     if (s->KM.alloc((size_t)s->nnz * 16) || (s->cplx && s->KMi.alloc((size_t)s->nnz * 16))) {
       (void)s->KM.alloc(0);  // no room: the padded kernels
@@ -3006,6 +3010,7 @@ extern "C" int efm_sweep_solve(efm_sweep *s, int nsys, const double *h_k0sq, con
       EFM_LAUNCH_CHECK();
     }
   }
+  s->last_flat = flat;
   // the wide kernels' system count is padded to whole wavefronts
   const int Bp = flat ? nsys : ((nsys + kSys - 1) / kSys) * kSys;
   const int P = s->P;

@@ -297,12 +297,13 @@ int efm_sweep_solve(efm_sweep *sw, int nsys, const double *h_k0sq, const double 
  * once per group of 64 systems into LDS and its rows read them there; available when
  * every tile fits (set returns an error otherwise); -1 (default) = with form 2, no
  * reliable updates and a batch that would leave many of its wavefronts' lanes idle (below
- * 40, 65-95 and 129-143 systems), kernels that pack the systems of several rows into a wavefront (get reports -1);
- * otherwise the fastest, chosen on the first solve: the iterations before its first convergence check cycle through the
- * candidates, each launch timed in place.  get: the variants in use (-1 before they are
- * chosen) and, when h_tune_ms is given (5 entries), the mean times in ms per launch
- * [SpMV 0, 1, 2, nodal 0, 1] (0 for a variant not timed).  Autotuner of this project; no
- * reference counterpart. */
+ * 40, 65-95 and 129-143 systems), kernels that pack the systems of several rows into a
+ * wavefront (get reports -1); otherwise the fastest, chosen on the first such solve: the
+ * iterations before its first convergence check cycle through the candidates, each launch
+ * timed in place.  The choice does not change which batches are packed.  get: the variants
+ * of the last solve (-1 before they are chosen) and, when h_tune_ms is given (5 entries),
+ * the mean times in ms per launch [SpMV 0, 1, 2, nodal 0, 1] (0 for a variant not timed).
+ * Autotuner of this project; no reference counterpart. */
 int efm_sweep_set_variants(efm_sweep *sw, int spmv, int aux);
 /* Iteration form of the batched COCG: 0 = standard COCG, p = u + beta p in a
  * streaming pass of its own and two reductions per iteration; 1 = Chronopoulos-Gear, one

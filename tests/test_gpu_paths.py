@@ -302,6 +302,44 @@ def test_packed_sweep_batches(torch_dev, nsys, levels, ring, lossy, graph):
     assert d <= 1e-9
 
 
+@pytest.mark.parametrize("graph", [False, True])
+def test_narrow_batch_after_a_wide_one(torch_dev, graph):
+    """A narrow batch on a sweep that has solved a wide one is packed as on a new sweep, with the
+    same bits, and a wide one after it runs what was chosen; pinned variants stay pinned."""
+    import torch
+    from edgefem_amd import _capi
+    xyz, tets = _fan_mesh(6, 24)
+    topo = _capi.Topology(np.arange(len(xyz)), tets, np.zeros((0, 3), np.int32))
+    n = topo.n_edges
+    rng = np.random.default_rng(3)
+    K, M = _capi.assemble_km(topo, xyz, np.full(len(tets), 2.0 - 0.3j))
+    k2 = -rng.uniform(1.0, 3.0, 128)
+    B = torch.from_numpy(rng.standard_normal((n, 128)) + 1j * rng.standard_normal((n, 128))).cuda()
+
+    def sweep():
+        s = _capi.SweepSolver(topo, K, M, [], None, 128)
+        s.set_graph(graph)
+        return s
+
+    def solve(s, m):
+        X, info = s.solve(k2[:m], np.zeros((m, 0)), B[:, :m].contiguous(), tol=1e-10, max_iterations=1000)
+        assert info["resid"].max() <= 1e-10
+        return X
+
+    ref = solve(sweep(), 18)
+    s = sweep()
+    solve(s, 128)
+    wide = s.variants()[:2]
+    assert min(wide) >= 0
+    X = solve(s, 18)
+    assert s.variants()[:2] == (-1, -1) and torch.equal(X, ref)
+    solve(s, 128)
+    assert s.variants()[:2] == wide
+    s.set_variants(1, 1)
+    solve(s, 18)
+    assert s.variants()[:2] == (1, 1)
+
+
 @pytest.mark.parametrize("n,nrhs,kind", [
     (5, 1, "real"), (511, 2, "mixed"), (512, 1, "complex"), (513, 2, "real"), (1600, 2, "mixed"), (9000, 1, "mixed"),
     (40000, 2, "scattered"), (3000, 2, "long")])
