@@ -1759,7 +1759,7 @@ constexpr int kZForm = 9;             // COCG with p formed in its own pass (its
 constexpr int kSellForm = 10;         // the same iteration with the sliced-ELL SpMV
 constexpr int kSplitForm = 11;        // the same iteration, values stored as real parts plus the imaginary parts of complex tiles
 constexpr int kSellRL = 4;            // lanes per row of the sliced-ELL SpMV
-constexpr int kPersistLaunch = 4096;  // iterations per launch at most
+constexpr int kPersistLaunch = 4096;  // iterations per launch at most, by default
 
 struct efm_solver {
   int64_t n = 0, nnz = 0;
@@ -1821,7 +1821,9 @@ struct efm_solver {
   efm::DevBuf lr_idx, lr_val, lr_coef;
   // persistent kernel (efm_persist.h), set up on first use: row blocks and their local columns
   int ncu = 256;
-  int ps_state = 0;  // 0: not tried, 1: set up, -1: the matrix does not fit
+  // 0: not tried, 1: set up, -1: the matrix does not fit, or a launch was refused or waited too long
+  int ps_state = 0;
+  int ps_launch = kPersistLaunch, ps_polls = efm_persist::kPolls;
   int ps_nb = 0, ps_rpb = 0, ps_nsm = 0, ps_lds = 0;
   bool ps_more = false;
   efm::DevBuf ps_lidx, ps_rloc, ps_ucol, ps_nu, ps_part, ps_cnt, ps_lrport, ps_lrw;
@@ -2500,6 +2502,7 @@ template <int R> struct Dispatch {
       a.p2 = s->W0.as<double2>();
       a.part = s->ps_part.as<double>();
       a.nsm = s->ps_nsm;
+      a.polls = s->ps_polls;
       a.cnt = s->ps_cnt.as<unsigned>();
       a.err = (int *)(s->ps_cnt.as<unsigned>() + kCounters * kCounterStride);
       a.lr_P = s->lr_P;
@@ -2523,7 +2526,7 @@ template <int R> struct Dispatch {
       Control *C = s->control.as<Control>();
       Control hc{};
       for (int its = 0; its < max_it;) {
-        int launch = std::min(max_it - its, kPersistLaunch);
+        int launch = std::min(max_it - its, s->ps_launch);
         double t2 = tol2;
         int mi = max_it;
         void *args[] = {&a, &S, &C, &launch, &t2, &mi};
@@ -2985,6 +2988,17 @@ extern "C" int efm_solver_get_spmv_variant(const efm_solver *s, int *h_variant, 
   return EFM_OK;
 }
 
+extern "C" int efm_solver_set_persist_limits(efm_solver *s, int launch_iterations, int polls) {
+  EFM_REQUIRE(s, "efm_solver_set_persist_limits: NULL solver");
+  EFM_REQUIRE(launch_iterations >= 0 && polls >= -1 && polls <= efm_persist::kPolls,
+              "efm_solver_set_persist_limits: limits out of range");
+  s->ps_launch = launch_iterations > 0 ? launch_iterations : kPersistLaunch;
+  s->ps_polls = polls >= 0 ? polls : efm_persist::kPolls;
+  if (s->ps_state < 0)
+    s->ps_state = 0;
+  return EFM_OK;
+}
+
 extern "C" int efm_solver_profile(efm_solver *s, int enable) {
   EFM_REQUIRE(s, "efm_solver_profile: NULL solver");
   s->profile = enable != 0;
@@ -3063,8 +3077,9 @@ extern "C" int efm_solver_solve(efm_solver *s, const double *B, double *X,
     });
     if (rc != EFM_OK)
       return rc;
-    if (!done) {  // from the start again, one launch per step
+    if (!done) {  // from the start again, one launch per step, and so from now on
       persist = false;
+      s->ps_state = -1;
       if ((rc = start()) != EFM_OK)
         return rc;
     }

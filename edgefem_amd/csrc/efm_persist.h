@@ -28,7 +28,7 @@
 // round trip with few blocks, 13.4 against 14.5 us per iteration with 4, and loses with many:
 // every block polls 12 words of every other, 22 against 19 us with 123.)
 //
-// Every wait ends: after kPollLimit polls a block gives up, sets the error flag and leaves,
+// Every wait ends: after Args::polls polls a block gives up, sets the error flag and leaves,
 // and so do the others; the caller then solves with one launch per step.  The launch is
 // cooperative, so all blocks are resident.  kRowsMin rows per block: 64 and 128 measured no
 // better at any size, as every block adds to the grid sums.
@@ -52,7 +52,7 @@ constexpr int kGroups = kThreads / kRL;    // rows per round
 constexpr int kJ = 6;                      // entries of a row per lane in registers
 constexpr int kCounters = 8;
 constexpr int kCounterStride = 32;         // uint32 per 128-byte line
-constexpr int kPollLimit = 1 << 21;        // a second or two
+constexpr int kPolls = 1 << 21;            // of one wait at most, by default: a second or two
 constexpr int kStage = 4;                  // staged columns per thread with their index in registers
 constexpr int kNodeLanes = 8;
 constexpr int kMaxLds = 150 * 1024;        // staged columns and LDS rows of a block
@@ -64,6 +64,7 @@ constexpr int kMaxD = 16;                  // doubles of a grid sum
 struct Args {
   int n, N, nb, rpb, npb;                  // rows, nodes, blocks, rows and nodes per block
   int nsm;                                 // most distinct columns of a block
+  int polls;                               // of one wait at most
   const int32_t *row_ptr, *col;
   const uint16_t *lidx, *rloc;             // local index of every entry's column, of every row
   const int32_t *ucol, *nu;                // distinct columns of block b at row_ptr[r0] + r0
@@ -331,13 +332,13 @@ __global__ void __launch_bounds__(kThreads)
     const int c = lane < kCounters ? lane : 0;
     const unsigned want = epoch * (unsigned)((a.nb - c + kCounters - 1) / kCounters);
     int k = 0;
-    for (; k < kPollLimit; ++k) {
+    for (; k < a.polls; ++k) {
       const unsigned v =
           __hip_atomic_load(a.cnt + c * kCounterStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (__all((int)(v - want) >= 0))
         break;
     }
-    if (k >= kPollLimit && lane == 0)
+    if (k >= a.polls && lane == 0)
       sh.err = 1;
   };
   auto wave_sum = [&](double &v) {

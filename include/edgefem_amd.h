@@ -204,6 +204,13 @@ int efm_solver_solve(efm_solver *s, const double *B, double *X, const efm_solve_
  * measured average ms per launch (-1 = not available).  No reference counterpart. */
 int efm_solver_set_spmv_variant(efm_solver *s, int variant);
 int efm_solver_get_spmv_variant(const efm_solver *s, int *h_variant, double *h_tune_ms);
+/* Limits of the persistent kernel: iterations per launch (0: the default, 4096) and polls of
+ * one wait of a block for the others (-1: the default, a second or two).  A solve whose
+ * launch is refused or whose blocks wait longer starts again with launches per step, and so
+ * does every later solve of this solver until the limits are set again.  Results do not
+ * depend on the iterations per launch (low-rank terms: to rounding).  No reference
+ * counterpart. */
+int efm_solver_set_persist_limits(efm_solver *s, int launch_iterations, int polls);
 
 /* y = A x (all nrhs systems), FP64 accumulation. */
 int efm_solver_spmv(efm_solver *s, const double *x, double *y, void *stream);

@@ -197,6 +197,86 @@ def test_systems_past_the_persistent_kernel(torch_dev, n, nrhs, dtype, terms):
     assert np.linalg.norm(r) <= (2e-10 if dtype == "complex128" else 1e-6) * np.linalg.norm(B)
 
 
+def _persistent_case(n, nrhs, aux, terms):
+    """Solver, right-hand sides (one of zeros) and what a residual needs."""
+    import torch
+    from edgefem_amd import _capi
+    A, en, B = _local_system(n, nrhs, n + 7, long_rows=(0, n - 1))
+    if nrhs > 1:
+        B[:, 0] = 0
+    lr = _lowrank_terms(n, terms, np.random.default_rng(n)) if terms else None
+
+    def solver():
+        s = _capi.KrylovSolver(A.indptr, A.indices, nrhs=nrhs)
+        if aux:
+            s.set_gradient(_Nodes(en))
+        if lr:
+            s.set_lowrank(lr[0].reshape(-1), lr[1].reshape(-1), lr[2])
+        s.set_matrix(A.data)
+        return s
+
+    def residual(X):
+        X = X.cpu().numpy().reshape(n, nrhs)
+        r = B - A @ X
+        for p in range(terms):
+            k = lr[0][p] >= 0
+            r[lr[0][p][k]] -= lr[2][p] * np.outer(lr[1][p][k], lr[1][p][k].conj() @ X[lr[0][p][k]])
+        return np.linalg.norm(r) / np.linalg.norm(B)
+
+    return solver, torch.from_numpy(B).cuda(), residual
+
+
+@pytest.mark.parametrize("n,nrhs,aux,terms", [
+    (700, 2, True, 0), (700, 2, True, 2), (700, 1, False, 3), (1100, 4, True, 0), (70000, 2, True, 1),
+    (70000, 1, False, 0)])
+@pytest.mark.parametrize("per_launch", [1, 5, 8])
+def test_persistent_kernel_over_several_launches(torch_dev, n, nrhs, aux, terms, per_launch):
+    """Iterations split over launches (odd and even numbers of them: p alternates between two
+    copies) are the ones of a single launch: bit for bit, with low-rank terms to the rounding
+    of w^H p, formed again at each launch (30 iterations of sums of 9 terms, below 1e-13 of x
+    times the condition number, below 10)."""
+    import torch
+    solver, b, residual = _persistent_case(n, nrhs, aux, terms)
+    for cap in (12, 1000):
+        one, many = solver(), solver()
+        many.set_persist_limits(per_launch)
+        X, i1 = one.solve(b, tol=1e-12, max_iterations=cap)
+        Y, i2 = many.solve(b, tol=1e-12, max_iterations=cap)
+        assert one.spmv_variant()[0] == many.spmv_variant()[0] == -1
+        if terms and cap == 1000:
+            assert i2["converged"] and residual(Y) <= 2e-12 and abs(max(i1["iters"]) - max(i2["iters"])) <= 1
+        else:
+            np.testing.assert_array_equal(i1["iters"], i2["iters"])
+        d = (X - Y).abs().max().item() / X.abs().max().item()
+        print(f"n {n} nrhs {nrhs} terms {terms} cap {cap}: iterations {i1['iters']} {i2['iters']} difference {d:.1e}",
+              flush=True)
+        assert d <= 1e-12 if terms else torch.equal(X, Y)
+
+
+@pytest.mark.parametrize("n,nrhs,aux,terms", [(700, 2, True, 0), (700, 1, False, 3), (70000, 2, True, 1)])
+def test_persistent_kernel_that_gives_up(torch_dev, n, nrhs, aux, terms):
+    """With no poll at all every block leaves its first wait at once: the solve starts again with
+    launches per step on the buffers that the kernel has written, and later solves of this
+    solver do not try it again, until the limits are set."""
+    import torch
+    solver, b, residual = _persistent_case(n, nrhs, aux, terms)
+    s, fresh = solver(), solver()
+    s.set_persist_limits(polls=0)
+    X, info = s.solve(b, tol=1e-12)
+    v = s.spmv_variant()[0]
+    assert v >= 0 and info["converged"] and residual(X) <= 2e-12
+    if nrhs > 1:
+        assert X.reshape(n, nrhs)[:, 0].abs().max().item() == 0
+    fresh.set_spmv_variant(v)
+    Y, _ = fresh.solve(b, tol=1e-12)
+    assert torch.equal(X, Y)
+    X, info = s.solve(b, tol=1e-12)
+    assert s.spmv_variant()[0] == v and torch.equal(X, Y)
+    s.set_persist_limits()
+    X, info = s.solve(b, tol=1e-12)
+    assert s.spmv_variant()[0] == -1 and info["converged"] and residual(X) <= 2e-12
+
+
 def test_tuned_solver_keeps_the_persistent_kernel(torch_dev):
     """A profiled solve and one with too many low-rank terms time the variants; what they chose does
     not change a later solve that the one kernel covers: the same bits as a fresh solver's."""
