@@ -2525,6 +2525,8 @@ template <int R> struct Dispatch {
       SysState *S = s->state.as<SysState>();
       Control *C = s->control.as<Control>();
       Control hc{};
+      int dev = 0;
+      EFM_HIP_CHECK(hipGetDevice(&dev));
       for (int its = 0; its < max_it;) {
         int launch = std::min(max_it - its, s->ps_launch);
         double t2 = tol2;
@@ -2532,6 +2534,7 @@ template <int R> struct Dispatch {
         void *args[] = {&a, &S, &C, &launch, &t2, &mi};
         int err = 0;
         EFM_HIP_CHECK(hipMemsetAsync(s->ps_cnt.p, 0, s->ps_cnt.bytes, st));
+        Gate gate(dev, s->ps_nb, s->ncu);
         if (hipLaunchCooperativeKernel(k, dim3(s->ps_nb), dim3(kThreads), args, s->ps_lds, st) != hipSuccess) {
           (void)hipGetLastError();
           return EFM_OK;

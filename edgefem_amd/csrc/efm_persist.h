@@ -28,6 +28,11 @@
 // round trip with few blocks, 13.4 against 14.5 us per iteration with 4, and loses with many:
 // every block polls 12 words of every other, 22 against 19 us with 123.)
 //
+// A block needs a CU to itself at most, and a launch has no more blocks than CUs.  Launches of
+// several threads on streams of their own could each get a part of the CUs and wait for
+// the rest, so a launch is admitted (Gate) while the blocks in flight on its device fit
+// on every XCD: block b of a launch runs on XCD b % 8.
+//
 // Every wait ends: after Args::polls polls a block gives up, sets the error flag and leaves,
 // and so do the others; the caller then solves with one launch per step.  The launch is
 // cooperative, so all blocks are resident.  kRowsMin rows per block: 64 and 128 measured no
@@ -39,6 +44,8 @@
 
 #include "efm_internal.h"
 
+#include <condition_variable>
+#include <mutex>
 #include <type_traits>
 
 namespace efm_persist {
@@ -103,6 +110,37 @@ __device__ inline void stc(Rsrc r, int i, double2 d) {
 }
 // every vector memory operation of this wave has completed
 __device__ inline void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
+// Launches in flight on a device of this process, each from its launch until its stream has ended
+// it.  The first to wait is the next to enter, so small launches do not pass a large one by.
+class Gate {
+  struct Device {
+    std::mutex turn, lock;
+    std::condition_variable left;
+    int used = 0;  // blocks per XCD
+  };
+  static Device &of(int dev) {
+    static Device d[64];
+    return d[dev & 63];
+  }
+  Device &d;
+  const int mine;
+
+public:
+  Gate(int dev, int blocks, int ncu) : d(of(dev)), mine((blocks + 7) / 8) {
+    std::lock_guard<std::mutex> t(d.turn);
+    std::unique_lock<std::mutex> l(d.lock);
+    d.left.wait(l, [&] { return d.used == 0 || d.used + mine <= ncu / 8; });
+    d.used += mine;
+  }
+  ~Gate() {
+    std::lock_guard<std::mutex> l(d.lock);
+    d.used -= mine;
+    d.left.notify_all();
+  }
+  Gate(const Gate &) = delete;
+  Gate &operator=(const Gate &) = delete;
+};
 
 // The scalars that a solve in separate launches keeps in memory (one system per lane).
 struct Scal {

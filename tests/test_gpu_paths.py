@@ -277,6 +277,34 @@ def test_persistent_kernel_that_gives_up(torch_dev, n, nrhs, aux, terms):
     assert s.spmv_variant()[0] == -1 and info["converged"] and residual(X) <= 2e-12
 
 
+def test_persistent_kernels_of_several_threads(torch_dev):
+    """Solvers whose blocks take all CUs, half of them and a few, in four threads on streams of
+    their own: no launch keeps another from its CUs (a wait that gave up would leave launches
+    per step), and every result is the one of a solver alone, bit for bit."""
+    import threading
+    import torch
+    sizes = [(65536, 1), (65400, 2), (30000, 2), (700, 2)]
+    cases = [_persistent_case(n, nrhs, False, 0) for n, nrhs in sizes]
+    ref = [solver().solve(b, tol=1e-12)[0] for solver, b, _ in cases]
+    solvers = [c[0]() for c in cases]
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(30):
+                X, _ = solvers[i].solve(cases[i][1], tol=1e-12)
+                if not torch.equal(X, ref[i]) or solvers[i].spmv_variant()[0] != -1:
+                    bad.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(cases))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+
+
 def test_tuned_solver_keeps_the_persistent_kernel(torch_dev):
     """A profiled solve and one with too many low-rank terms time the variants; what they chose does
     not change a later solve that the one kernel covers: the same bits as a fresh solver's."""
