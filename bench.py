@@ -785,6 +785,7 @@ def main():
     te = time.perf_counter()
     spmv_ms, spmv_n = pipe.solver.profile_read()
     variant, tune_ms = pipe.solver.spmv_variant()
+    staged = pipe.solver.staged()
     pipe.solver.profile(False)
     elapsed = te - ts
     ms_per_step = 1e3 * elapsed / args.steps
@@ -837,7 +838,7 @@ def main():
                    "mode": args.mode},
         "roofline": {"bound": "hbm", "achieved": achieved / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK, "traffic": traffic, "traffic_unit": "GB per launch",
-                     "kernel": {9: "k_cocgz_spmv", 10: "k_cocgz_sell", 11: "k_staged (columns of 512 rows in LDS)"}.get(variant, "k_cocg_spmv"),
+                     "kernel": {9: "k_cocgz_spmv", 10: "k_cocgz_sell", 11: "k_staged (columns of 512 rows in LDS)" if staged else "k_cocgz_spmv (split values)"}.get(variant, "k_cocg_spmv"),
                      "bytes_per_launch": spmv_bytes, "avg_launch_ms": avg_ms, "launches": spmv_n,
                      "variant": variant, "autotune_ms": [round(float(t), 4) for t in tune_ms]},
         "cpu_baseline": cpu,

@@ -38,7 +38,7 @@ EXPORTS = [
     "efm_touchstone_write", "efm_touchstone_write_2port", "efm_touchstone_extension",
     "efm_port_overlap_noalloc", "efm_sweep_set_graph", "efm_sweep_set_correction",
     "efm_sweep_set_correction_values", "efm_sweep_set_correction_terms", "efm_direct_solve",
-    "efm_solver_set_persist_limits", "efm_array_package_json", "efm_patterns_csv", "efm_coupling_csv", "efm_scan_csv",
+    "efm_solver_set_persist_limits", "efm_solver_get_staged", "efm_array_package_json", "efm_patterns_csv", "efm_coupling_csv", "efm_scan_csv",
 ]
 
 
@@ -105,6 +105,7 @@ def load_library(path: str = LIB_PATH) -> C.CDLL:
     lib.efm_solver_profile_read.argtypes = [vp, C.POINTER(C.c_double), C.POINTER(C.c_int64)]
     lib.efm_solver_set_spmv_variant.argtypes = [vp, i32]
     lib.efm_solver_get_spmv_variant.argtypes = [vp, C.POINTER(C.c_int), vp]
+    lib.efm_solver_get_staged.argtypes = [vp, C.POINTER(C.c_int)]
     lib.efm_solver_set_persist_limits.argtypes = [vp, i32, i32]
     lib.efm_sweep_create.argtypes = [vp, vp, vp, i32, vp, vp, i32, vp, C.POINTER(vp)]
     lib.efm_solver_set_lowrank.argtypes = [vp, i32, C.c_int64, vp, vp, vp, vp]
@@ -414,6 +415,12 @@ class KrylovSolver:
         _check(self._lib.efm_solver_get_spmv_variant(self._h, C.byref(v), ms.ctypes.data_as(C.c_void_p)),
                "efm_solver_get_spmv_variant")
         return v.value, ms
+
+    def staged(self) -> bool:
+        """Whether the SpMV of the last solve was variant 11 with its columns staged in LDS."""
+        v = C.c_int()
+        _check(self._lib.efm_solver_get_staged(self._h, C.byref(v)), "efm_solver_get_staged")
+        return bool(v.value)
 
     def set_persist_limits(self, launch_iterations: int = 0, polls: int = -1):
         """Iterations per launch of the persistent kernel and polls of one of its waits (0 and

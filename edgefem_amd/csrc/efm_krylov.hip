@@ -2991,6 +2991,12 @@ extern "C" int efm_solver_get_spmv_variant(const efm_solver *s, int *h_variant, 
   return EFM_OK;
 }
 
+extern "C" int efm_solver_get_staged(const efm_solver *s, int *h_staged) {
+  EFM_REQUIRE(s && h_staged, "efm_solver_get_staged: NULL argument");
+  *h_staged = s->spmv_variant == kSplitForm && !s->last_persist && s->st_state > 0;
+  return EFM_OK;
+}
+
 extern "C" int efm_solver_set_persist_limits(efm_solver *s, int launch_iterations, int polls) {
   EFM_REQUIRE(s, "efm_solver_set_persist_limits: NULL solver");
   EFM_REQUIRE(launch_iterations >= 0 && polls >= -1 && polls <= efm_persist::kPolls,

@@ -204,6 +204,8 @@ int efm_solver_solve(efm_solver *s, const double *B, double *X, const efm_solve_
  * measured average ms per launch (-1 = not available).  No reference counterpart. */
 int efm_solver_set_spmv_variant(efm_solver *s, int variant);
 int efm_solver_get_spmv_variant(const efm_solver *s, int *h_variant, double *h_tune_ms);
+/* 1 where the SpMV of the last solve was variant 11 with its columns staged in LDS. */
+int efm_solver_get_staged(const efm_solver *s, int *h_staged);
 /* Limits of the persistent kernel: iterations per launch (0: the default, 4096) and polls of
  * one wait of a block for the others (-1: the default, a second or two).  A solve whose
  * launch is refused or whose blocks wait longer starts again with launches per step, and so

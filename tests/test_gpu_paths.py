@@ -493,8 +493,26 @@ def test_staged_spmv_tiles(torch_dev, n, nrhs, kind):
                 rel = (np.linalg.norm(B - Am @ X[variant, cap], axis=0) / np.linalg.norm(B, axis=0)).max()
                 print(f"n {n} {kind}: iterations {max(info['iters'])} true {rel:.1e}", flush=True)
                 assert info["converged"] and rel <= 2e-12
+                assert s.staged() == (kind != "scattered")
         d = np.abs(X[11, 7] - X[0, 7]).max() / np.abs(X[0, 7]).max()
         assert d <= max(1e-13, n * 2.3e-16), d
+        assert not s.staged()   # variant 0 ran last
+
+
+def test_staged_spmv_needs_few_right_hand_sides(torch_dev):
+    """With three right-hand sides variant 11 runs on split values, and the persistent kernel is
+    not reported as staged."""
+    import torch
+    from edgefem_amd import _capi
+    for nrhs, variant, staged in ((3, 11, False), (2, 11, True), (2, -1, False)):
+        A, en, B = _local_system(900, nrhs, 5)
+        s = _capi.KrylovSolver(A.indptr, A.indices, nrhs=nrhs)
+        s.set_gradient(_Nodes(en))
+        s.set_matrix(A.data)
+        s.set_spmv_variant(variant)
+        X, info = s.solve(torch.from_numpy(B).cuda(), tol=1e-12)
+        rel = np.linalg.norm(B - A @ X.cpu().numpy().reshape(B.shape)) / np.linalg.norm(B)
+        assert info["converged"] and rel <= 2e-12 and s.staged() == staged
 
 
 @pytest.mark.parametrize("grid", [1, 3, 4, 6, 9, 10])
