@@ -2074,8 +2074,11 @@ template <int R> struct Dispatch {
         return EFM_OK;
       }
       EFM_HIP_CHECK(hipMemcpyAsync(s->st_steps.p, steps.data(), nw * sizeof(int2), hipMemcpyHostToDevice, st));
-      const void *k = reinterpret_cast<const void *>(&k_index);
-      EFM_HIP_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, words * 8));
+      // the limits belong to the kernels, not to this solver: the most that any solver may ask for
+      EFM_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_index),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, kMaxWords * 8));
+      EFM_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&efm_staged::k_staged<R, SysState>),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, efm_staged::kMaxLds));
       hipLaunchKernelGGL(k_index, dim3((unsigned)nt), dim3(kTile), words * 8, st, (int)n, words, cap, s->row_ptr,
                          s->col, s->st_srow.as<uint16_t>(), s->st_steps.as<int2>(), window.as<int2>(),
                          s->st_ucol.as<int32_t>(), s->st_nu.as<int32_t>(), s->st_sown.as<uint16_t>(),
@@ -2092,8 +2095,6 @@ template <int R> struct Dispatch {
       s->st_cap = cap;
       s->st_lds = *std::max_element(nu.begin(), nu.end()) * R * (int)sizeof(double2);
       s->st_pairs = total;
-      EFM_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(&efm_staged::k_staged<R, SysState>),
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, s->st_lds));
       s->st_state = 1;
     }
     if (s->st_state < 0)
@@ -2521,7 +2522,8 @@ template <int R> struct Dispatch {
       const std::true_type T{};
       const std::false_type F{};
       const void *k = s->aux ? (lr ? pick(T, T) : pick(T, F)) : (lr ? pick(F, T) : pick(F, F));
-      EFM_HIP_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, s->ps_lds));
+      // the same value from every solver: the limit belongs to the kernel
+      EFM_HIP_CHECK(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds));
       SysState *S = s->state.as<SysState>();
       Control *C = s->control.as<Control>();
       Control hc{};

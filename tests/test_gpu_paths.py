@@ -499,6 +499,46 @@ def test_staged_spmv_tiles(torch_dev, n, nrhs, kind):
         assert not s.staged()   # variant 0 ran last
 
 
+def _spread_system(n, reach, nrhs, seed):
+    """A diagonally dominant matrix whose rows couple up to `reach` away, eight entries to a side."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(seed)
+    i = np.repeat(np.arange(n), 8)
+    j = i + rng.integers(1, reach, i.size)
+    ok = j < n
+    off = sp.csr_matrix((rng.standard_normal(ok.sum()) + 0.1j, (i[ok], j[ok])), shape=(n, n))
+    off = off + off.T
+    A = (off + sp.diags(np.asarray(abs(off).sum(axis=1)).ravel() * 1.6 + 1.0)).tocsr()
+    A.sort_indices()
+    return A, rng.standard_normal((n, nrhs)) + 1j * rng.standard_normal((n, nrhs))
+
+
+def test_staged_solvers_of_different_tiles(torch_dev):
+    """The LDS limit of a kernel belongs to all solvers: one of large tiles (more than 64 KiB of
+    columns) solves before and after another of small ones is built, with the same bits."""
+    import torch
+    from edgefem_amd import _capi
+
+    def make(reach):
+        A, B = _spread_system(4000, reach, 2, reach)
+        s = _capi.KrylovSolver(A.indptr, A.indices, nrhs=2)
+        s.set_matrix(A.data)
+        s.set_spmv_variant(11)
+        tiles = [A[r:r + 512] for r in range(0, 4000, 512)]
+        return s, torch.from_numpy(B).cuda(), max(np.unique(t.indices).size for t in tiles) * 32
+
+    large, b, lds = make(1000)
+    assert 65536 < lds < 80 * 1024
+    X, info = large.solve(b, tol=1e-12)
+    assert info["converged"] and large.staged()
+    small, b2, lds = make(40)
+    assert lds < 32768
+    Y, info = small.solve(b2, tol=1e-12)
+    assert info["converged"] and small.staged()
+    X2, info = large.solve(b, tol=1e-12)
+    assert info["converged"] and large.staged() and torch.equal(X, X2)
+
+
 def test_staged_spmv_needs_few_right_hand_sides(torch_dev):
     """With three right-hand sides variant 11 runs on split values, and the persistent kernel is
     not reported as staged."""
