@@ -32,7 +32,9 @@ using namespace efm;
 constexpr int kTile = 512;                // rows of a tile, threads of a block
 constexpr int kWavesT = kTile / 64;
 constexpr int kPre = 2;                   // pairs of a row loaded at a time, two groups ahead
-constexpr int kMaxLds = 80 * 1024;        // staged columns: two blocks per CU
+constexpr int kMostRhs = 2;
+constexpr int kRedBytes = kWavesT * kMostRhs * 16;
+constexpr int kMaxLds = 80 * 1024 - kRedBytes;  // staged columns: with the sums' LDS, two blocks per CU
 constexpr int kMaxWords = 16384;          // words of the window of columns of a tile
 constexpr int kMaxLen = 255;              // entries of a row
 
@@ -182,6 +184,7 @@ __global__ void __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(6, 8
            double2 *__restrict__ q, double2 *__restrict__ partial, const State *__restrict__ st) {
   extern __shared__ double2 xs[];
   __shared__ double2 red[kWavesT][R];
+  static_assert(R <= kMostRhs && sizeof(red) <= kRedBytes, "two blocks per CU");
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
   const int lb = blockIdx.x >> 3, tile = (blockIdx.x & 7) * xcd_span + lb;
   double2 pq[R];

@@ -539,6 +539,30 @@ def test_staged_solvers_of_different_tiles(torch_dev):
     assert info["converged"] and large.staged() and torch.equal(X, X2)
 
 
+@pytest.mark.parametrize("nrhs", [1, 2])
+def test_staged_tile_at_the_most_columns(torch_dev, nrhs):
+    """The first tile reads exactly the columns that leave room for two blocks in the 160 KiB of a
+    CU (80 KiB less 16 bytes per wavefront and right-hand side of two), and one more: staged and
+    not, both solved."""
+    import scipy.sparse as sp
+    import torch
+    from edgefem_amd import _capi
+    most = (80 * 1024 - 8 * 2 * 16) // (16 * nrhs)
+    rng = np.random.default_rng(nrhs)
+    for cols in (most, most + 1):
+        extra, n = cols - 512, cols + 100
+        off = sp.csr_matrix((np.full(extra, 0.2 + 0.1j), (np.arange(extra) % 512, 512 + np.arange(extra))), shape=(n, n))
+        A = (off + off.T + sp.diags(np.full(n, 4.0 + 1j))).tocsr()
+        A.sort_indices()
+        B = rng.standard_normal((n, nrhs)) + 1j * rng.standard_normal((n, nrhs))
+        s = _capi.KrylovSolver(A.indptr, A.indices, nrhs=nrhs)
+        s.set_matrix(A.data)
+        s.set_spmv_variant(11)
+        X, info = s.solve(torch.from_numpy(B).cuda(), tol=1e-12)
+        rel = np.linalg.norm(B - A @ X.cpu().numpy().reshape(B.shape)) / np.linalg.norm(B)
+        assert info["converged"] and rel <= 2e-12 and s.staged() == (cols == most)
+
+
 def test_staged_spmv_needs_few_right_hand_sides(torch_dev):
     """With three right-hand sides variant 11 runs on split values, and the persistent kernel is
     not reported as staged."""
