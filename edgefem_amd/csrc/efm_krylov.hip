@@ -2418,27 +2418,29 @@ template <int R> struct Dispatch {
       s->ps_state = -1;
       const int64_t n = s->n;
       constexpr int most = max_rows(R <= 2);
-      if (s->vtype != EFM_C128 || n > (int64_t)s->ncu * most)
+      if (s->vtype != EFM_C128 || n > (int64_t)s->ncu * most || s->nnz > kMaxMean * n)
         return EFM_OK;
       const int64_t rpb = std::max<int64_t>(kRowsMin, (n + s->ncu - 1) / s->ncu);
       const int nb = (int)((n + rpb - 1) / rpb);
       if (s->ps_lidx.alloc((size_t)s->nnz * 2) || s->ps_rloc.alloc((size_t)n * 2) ||
-          s->ps_ucol.alloc((size_t)(s->nnz + n) * 4) || s->ps_nu.alloc((size_t)nb * 4) ||
+          s->ps_ucol.alloc((size_t)(s->nnz + n) * 4) || s->ps_nu.alloc((size_t)2 * nb * 4) ||
           s->ps_part.alloc((size_t)3 * nb * kMaxD * 8) ||
           s->ps_cnt.alloc((size_t)kCounters * kCounterStride * 4 + 128))
         return EFM_OK;  // no room: one launch per step
       const size_t lds = (size_t)2 * ((n + 31) / 32) * 4;
       hipLaunchKernelGGL(k_persist_cols, dim3(nb), dim3(kThreads), lds, st, (int)n, (int)rpb, s->row_ptr, s->col,
                          s->ps_lidx.as<uint16_t>(), s->ps_rloc.as<uint16_t>(), s->ps_ucol.as<int32_t>(),
-                         s->ps_nu.as<int32_t>());
+                         s->ps_nu.as<int32_t>(), s->ps_nu.as<int32_t>() + nb);
       EFM_LAUNCH_CHECK();
-      std::vector<int32_t> nu(nb), rp(s->n + 1);
-      EFM_HIP_CHECK(hipMemcpyAsync(nu.data(), s->ps_nu.p, (size_t)nb * 4, hipMemcpyDeviceToHost, st));
+      std::vector<int32_t> nu(2 * nb), rp(s->n + 1);  // columns of the blocks, then their longest rows
+      EFM_HIP_CHECK(hipMemcpyAsync(nu.data(), s->ps_nu.p, (size_t)2 * nb * 4, hipMemcpyDeviceToHost, st));
       const bool more = rpb > max_rows(false);
       if (more)
         EFM_HIP_CHECK(hipMemcpyAsync(rp.data(), s->row_ptr, (size_t)(n + 1) * 4, hipMemcpyDeviceToHost, st));
       EFM_HIP_CHECK(hipStreamSynchronize(st));
-      const int mx = *std::max_element(nu.begin(), nu.end());
+      const int mx = *std::max_element(nu.begin(), nu.begin() + nb);
+      if (*std::max_element(nu.begin() + nb, nu.end()) > kMaxRow)
+        return EFM_OK;
       int64_t need = (int64_t)mx * R * sizeof(double2), entries = 0;
       if (more)
         for (int64_t r = 0; r < n; r += rpb)

@@ -65,6 +65,12 @@ constexpr int kNodeLanes = 8;
 constexpr int kMaxLds = 150 * 1024;        // staged columns and LDS rows of a block
 constexpr int kKR = 2;                     // rows per lane group in registers
 constexpr int kRowsMin = 256;              // rows per block at least (fewer only add blocks to each grid sum)
+// Entries of the longest row, and of a row on average, at most.  Entries past a lane group's
+// registers are a serial walk through memory, which the other blocks wait for at the next sum.
+// us per iteration with one right-hand side, launches per step against this: 31 k rows of 16 with
+// one of 256 17, 14, of 512 20, 21, of 1,000 24, 32; 31 k rows of 91 on average (118 at most) 27,
+// 24, of 150 (186) 27, 36.
+constexpr int kMaxRow = 256, kMaxMean = 96;
 constexpr int kMaxLr = 4;                  // low-rank terms times right-hand sides
 constexpr int kMaxD = 16;                  // doubles of a grid sum
 
@@ -151,26 +157,32 @@ struct Scal {
 
 // Distinct columns of every block's rows (and the rows themselves), ascending, and the local
 // index of every entry: a bitmap of all columns in LDS, ranks by prefix sums of its words.
+// longest: entries of the block's longest row.
 // One block of kThreads per row block; dynamic LDS 2 * words uint32.
 __global__ void __launch_bounds__(kThreads)
     k_persist_cols(int n, int rpb, const int32_t *__restrict__ row_ptr, const int32_t *__restrict__ col,
                    uint16_t *__restrict__ lidx, uint16_t *__restrict__ rloc, int32_t *__restrict__ ucol,
-                   int32_t *__restrict__ nu) {
+                   int32_t *__restrict__ nu, int32_t *__restrict__ longest) {
   extern __shared__ uint32_t sm[];
   const int words = (n + 31) / 32;
   uint32_t *bits = sm, *pre = sm + words;
   __shared__ uint32_t wsum[kThreads];
+  __shared__ int mx;
   const int r0 = blockIdx.x * rpb, r1 = min(n, r0 + rpb);
   const int32_t k0 = row_ptr[r0], k1 = row_ptr[r1];
   for (int w = threadIdx.x; w < words; w += kThreads)
     bits[w] = 0;
+  if (threadIdx.x == 0)
+    mx = 0;
   __syncthreads();
   for (int32_t k = k0 + threadIdx.x; k < k1; k += kThreads) {
     const int32_t c = col[k];
     atomicOr(&bits[c >> 5], 1u << (c & 31));
   }
-  for (int r = r0 + threadIdx.x; r < r1; r += kThreads)
+  for (int r = r0 + threadIdx.x; r < r1; r += kThreads) {
     atomicOr(&bits[r >> 5], 1u << (r & 31));
+    atomicMax(&mx, row_ptr[r + 1] - row_ptr[r]);
+  }
   __syncthreads();
   const int per = (words + kThreads - 1) / kThreads;
   const int w0 = min(words, (int)threadIdx.x * per), w1 = min(words, w0 + per);
@@ -197,8 +209,10 @@ __global__ void __launch_bounds__(kThreads)
       b &= b - 1;
     }
   }
-  if (threadIdx.x == 0)
+  if (threadIdx.x == 0) {
     nu[blockIdx.x] = (int32_t)wsum[kThreads - 1];
+    longest[blockIdx.x] = mx;
+  }
   __syncthreads();
   auto rank = [&](int32_t c) {
     return (uint16_t)(pre[c >> 5] + __popc(bits[c >> 5] & ((1u << (c & 31)) - 1)));

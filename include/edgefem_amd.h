@@ -195,7 +195,8 @@ int efm_solver_solve(efm_solver *s, const double *B, double *X, const efm_solve_
  * matrices; rebuilt on the device after every set_matrix), and, with one or two right-hand
  * sides where the columns of every 512 rows fit, those columns staged in LDS.  By
  * default (-1) complex-double COCG solves of up to 512 rows per CU (256 with three or four
- * right-hand sides; at most four low-rank terms times right-hand sides) run in one
+ * right-hand sides; at most four low-rank terms times right-hand sides; rows of at most 256
+ * entries, 96 on average) run in one
  * persistent kernel that keeps the matrix in registers and LDS (get reports -1); the first
  * other solve (a profiled one, too) times variants 0-11 on the installed matrix and keeps
  * the fastest for solves of its kind; a fixed variant makes results reproducible bit for

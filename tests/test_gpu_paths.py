@@ -197,6 +197,39 @@ def test_systems_past_the_persistent_kernel(torch_dev, n, nrhs, dtype, terms):
     assert np.linalg.norm(r) <= (2e-10 if dtype == "complex128" else 1e-6) * np.linalg.norm(B)
 
 
+@pytest.mark.parametrize("kind,rows,entries,one_kernel", [
+    ("one long row", 1500, 256, True), ("one long row", 1500, 257, False), ("one long row", 1500, 1100, False),
+    ("all rows", 900, 96, True), ("all rows", 900, 97, False)])
+def test_persistent_kernel_by_row_length(torch_dev, kind, rows, entries, one_kernel):
+    """The longest row and the mean row at their limits and one entry past them; longer rows go to
+    the timed variants, as before there was one kernel.  Tolerance as in test_persistent_cocg_edges."""
+    import scipy.sparse as sp
+    import torch
+    from edgefem_amd import _capi
+    rng = np.random.default_rng(entries)
+    k = np.arange(rows)
+    if kind == "all rows":   # a ring of `entries` columns centred on the row (one more past it where even)
+        off = [d for d in range(1, (entries - 1) // 2 + 1)]
+        A = sum(sp.csr_matrix((np.full(rows, 0.1 + 0.02j), (k, (k + d) % rows)), shape=(rows, rows)) for d in off)
+        A = A + A.T
+        if entries % 2 == 0:
+            A = A + sp.csr_matrix((np.full(rows, 0.1), (k, (k + rows // 2) % rows)), shape=(rows, rows))
+    else:
+        r = rows // 2
+        j = np.delete(np.arange(r - entries // 2, r - entries // 2 + entries), entries // 2)
+        A = sp.csr_matrix((np.full(entries - 1, 0.05 + 0.01j), (np.full(entries - 1, r), j)), shape=(rows, rows))
+        A = A + A.T
+    A = (A + sp.diags(np.asarray(abs(A).sum(axis=1)).ravel() * 1.6 + 1.0)).tocsr()
+    A.sort_indices()
+    assert np.diff(A.indptr).max() == entries and (kind != "all rows" or A.nnz == rows * entries)
+    B = rng.standard_normal((rows, 2)) + 1j * rng.standard_normal((rows, 2))
+    s = _capi.KrylovSolver(A.indptr, A.indices, nrhs=2)
+    s.set_matrix(A.data)
+    X, info = s.solve(torch.from_numpy(B).cuda(), tol=1e-12)
+    rel = np.linalg.norm(B - A @ X.cpu().numpy().reshape(B.shape)) / np.linalg.norm(B)
+    assert info["converged"] and rel <= 2e-12 and (s.spmv_variant()[0] == -1) == one_kernel
+
+
 def _persistent_case(n, nrhs, aux, terms):
     """Solver, right-hand sides (one of zeros) and what a residual needs."""
     import torch
