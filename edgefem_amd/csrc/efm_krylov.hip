@@ -2042,8 +2042,10 @@ template <int R> struct Dispatch {
         return EFM_OK;
       DevBuf pairs, window, bad;
       if (pairs.alloc((size_t)nw * 4) || window.alloc((size_t)nt * sizeof(int2)) || bad.alloc(sizeof(int)) ||
-          s->st_srow.alloc((size_t)nt * kTile * 2))
+          s->st_srow.alloc((size_t)nt * kTile * 2)) {
+        drop_staged(s);  // no room: the split values as before
         return EFM_OK;
+      }
       EFM_HIP_CHECK(hipMemsetAsync(bad.p, 0, sizeof(int), st));
       hipLaunchKernelGGL(k_order, dim3((unsigned)nt), dim3(kTile), 0, st, (int)n, s->row_ptr, s->col,
                          s->st_srow.as<uint16_t>(), pairs.as<int32_t>(), window.as<int2>(), bad.as<int>());
@@ -2063,14 +2065,16 @@ template <int R> struct Dispatch {
       int words = 0;
       for (const int2 &w : hw)
         words = std::max(words, (w.y - (w.x & ~31)) / 32 + 1);
-      if (hbad || words > kMaxWords || total >= INT32_MAX)
+      if (hbad || words > kMaxWords || total >= INT32_MAX) {
+        drop_staged(s);
         return EFM_OK;
+      }
       // one step more than is stored: a wavefront without rows at the end reads it, unused
       if (s->st_steps.alloc((size_t)nw * sizeof(int2)) || s->st_sown.alloc((size_t)nt * kTile * 2) ||
           s->st_ucol.alloc((size_t)nt * cap * 4) || s->st_nu.alloc((size_t)nt * 4) ||
           s->st_idx.alloc((size_t)(total + 1) * 64 * 4) || s->st_iflag.alloc((size_t)nt * 4) ||
           s->st_re.alloc((size_t)(total + 1) * 64 * 16)) {
-        drop_staged(s);  // no room: the split values as before
+        drop_staged(s);
         return EFM_OK;
       }
       EFM_HIP_CHECK(hipMemcpyAsync(s->st_steps.p, steps.data(), nw * sizeof(int2), hipMemcpyHostToDevice, st));
@@ -2411,6 +2415,13 @@ template <int R> struct Dispatch {
   }
 
   // ---- persistent form --------------------------------------------------------------------
+  static void drop_persist(efm_solver *s) {
+    for (DevBuf *b : {&s->ps_lidx, &s->ps_rloc, &s->ps_ucol, &s->ps_nu, &s->ps_part, &s->ps_cnt, &s->ps_lrport,
+                      &s->ps_lrw})
+      (void)b->alloc(0);
+    s->ps_lr_ok = false;
+    s->ps_state = -1;
+  }
   // Row blocks and local columns; s->ps_state says whether the matrix fits.
   static int persist_setup(efm_solver *s, hipStream_t st) {
     if constexpr (R <= 4) {
@@ -2425,8 +2436,10 @@ template <int R> struct Dispatch {
       if (s->ps_lidx.alloc((size_t)s->nnz * 2) || s->ps_rloc.alloc((size_t)n * 2) ||
           s->ps_ucol.alloc((size_t)(s->nnz + n) * 4) || s->ps_nu.alloc((size_t)2 * nb * 4) ||
           s->ps_part.alloc((size_t)3 * nb * kMaxD * 8) ||
-          s->ps_cnt.alloc((size_t)kCounters * kCounterStride * 4 + 128))
-        return EFM_OK;  // no room: one launch per step
+          s->ps_cnt.alloc((size_t)kCounters * kCounterStride * 4 + 128)) {
+        drop_persist(s);  // no room: one launch per step
+        return EFM_OK;
+      }
       const size_t lds = (size_t)2 * ((n + 31) / 32) * 4;
       hipLaunchKernelGGL(k_persist_cols, dim3(nb), dim3(kThreads), lds, st, (int)n, (int)rpb, s->row_ptr, s->col,
                          s->ps_lidx.as<uint16_t>(), s->ps_rloc.as<uint16_t>(), s->ps_ucol.as<int32_t>(),
@@ -2439,15 +2452,15 @@ template <int R> struct Dispatch {
         EFM_HIP_CHECK(hipMemcpyAsync(rp.data(), s->row_ptr, (size_t)(n + 1) * 4, hipMemcpyDeviceToHost, st));
       EFM_HIP_CHECK(hipStreamSynchronize(st));
       const int mx = *std::max_element(nu.begin(), nu.begin() + nb);
-      if (*std::max_element(nu.begin() + nb, nu.end()) > kMaxRow)
-        return EFM_OK;
       int64_t need = (int64_t)mx * R * sizeof(double2), entries = 0;
       if (more)
         for (int64_t r = 0; r < n; r += rpb)
           entries = std::max<int64_t>(entries, rp[std::min(n, r + rpb)] - rp[std::min(n, r + max_rows(false))]);
       need += entries * (sizeof(double2) + 2) + 16;
-      if (mx > 65535 || need > kMaxLds)
+      if (mx > 65535 || need > kMaxLds || *std::max_element(nu.begin() + nb, nu.end()) > kMaxRow) {
+        drop_persist(s);
         return EFM_OK;
+      }
       s->ps_nb = nb;
       s->ps_rpb = (int)rpb;
       s->ps_more = more;
@@ -2484,7 +2497,6 @@ template <int R> struct Dispatch {
       a.rpb = s->ps_rpb;
       a.npb = s->aux ? (int)((s->n_nodes + s->ps_nb - 1) / s->ps_nb) : 0;
       a.row_ptr = s->row_ptr;
-      a.col = s->col;
       a.lidx = s->ps_lidx.as<uint16_t>();
       a.rloc = s->ps_rloc.as<uint16_t>();
       a.ucol = s->ps_ucol.as<int32_t>();
@@ -3092,7 +3104,7 @@ extern "C" int efm_solver_solve(efm_solver *s, const double *B, double *X,
       return rc;
     if (!done) {  // from the start again, one launch per step, and so from now on
       persist = false;
-      s->ps_state = -1;
+      Dispatch<1>::drop_persist(s);
       if ((rc = start()) != EFM_OK)
         return rc;
     }

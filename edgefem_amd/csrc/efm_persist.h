@@ -78,7 +78,7 @@ struct Args {
   int n, N, nb, rpb, npb;                  // rows, nodes, blocks, rows and nodes per block
   int nsm;                                 // most distinct columns of a block
   int polls;                               // of one wait at most
-  const int32_t *row_ptr, *col;
+  const int32_t *row_ptr;
   const uint16_t *lidx, *rloc;             // local index of every entry's column, of every row
   const int32_t *ucol, *nu;                // distinct columns of block b at row_ptr[r0] + r0
   const double2 *val, *dinv;

@@ -1975,9 +1975,8 @@ __device__ inline int gsign_of(const int32_t *__restrict__ en, int32_t e, int32_
   return (node == b) ? 1 : ((node == a) ? -1 : 0);
 }
 
-// one thread per node: diag(G^T X G) for X in {K, M, Ms_p} (Dirichlet edges dropped)
-// kDiagLanes lanes per node, one incident edge per lane at a time: 39 us (one thread per node 261
-// us) for 7 k nodes.
+// diag(G^T X G) for X in {K, M, Ms_p} (Dirichlet edges dropped): kDiagLanes lanes per node, one
+// incident edge per lane at a time.  39 us for 7 k nodes (one thread per node: 261).
 constexpr int kDiagLanes = 16;
 __global__ void __launch_bounds__(kBlock)
     k_sw_node_diag(int64_t N, int P, const int32_t *__restrict__ n2e_ptr, const int32_t *__restrict__ n2e,
