@@ -251,8 +251,8 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
-// The scratch of one assembly: the topology's, or its own where another call holds that.  The
-// work that uses it has ended when it is given back.
+// The scratch of one assembly: the topology's, or its own where another call holds that or where it
+// is too large to keep.  The work that uses it has ended when it is given back.
 struct ElementScratch {
   const efm_topology *topo;
   hipStream_t st;
@@ -270,7 +270,7 @@ struct ElementScratch {
   int get(double2 **out) {
     const size_t bytes = (size_t)topo->T * 21 * sizeof(double2) + 16;
     std::lock_guard<std::mutex> g(topo->km_lock);
-    kept = !topo->km_held;
+    kept = !topo->km_held && bytes <= efm_topology::kKeepKm;
     DevBuf &b = kept ? topo->km : own;
     if (!b.p) {
       const int rc = b.alloc(bytes);

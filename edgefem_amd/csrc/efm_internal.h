@@ -67,8 +67,10 @@ struct efm_topology {
   efm::DevBuf n2e_ptr;    // int32 [N+1]   node -> incident edges, ascending
   efm::DevBuf n2e;        // int32 [2*n_edges]
   // element blocks of an assembly (336 B per tet), kept for the next one: an allocation and a
-  // free of 129 MB took 291 us of an assembly of 384 k tets (2.15 ms, now 1.85).  One call at a time holds it; a call
-  // from another thread meanwhile allocates its own.
+  // free of 129 MB took 291 us of an assembly of 384 k tets (2.15 ms, now 1.85).  Kept up to kKeepKm
+  // bytes (3.2 M tets): beyond, a mesh would hold what its solver may need.  One call at a
+  // time holds it; a call from another thread meanwhile allocates its own.
+  static constexpr size_t kKeepKm = (size_t)1 << 30;
   mutable std::mutex km_lock;
   mutable bool km_held = false;
   mutable efm::DevBuf km;

@@ -666,3 +666,35 @@ def test_assembly_scratch_from_two_threads(torch_dev):
     for t in threads:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("levels,keeps", [(20000, True), (65000, False)])
+def test_assembly_scratch_is_bounded(torch_dev, levels, keeps):
+    """An assembly's scratch (336 bytes per tet) stays with the mesh up to 1 GiB and is freed beyond:
+    what the device has less after an assembly, apart from torch's own pool, is the scratch (320 MiB)
+    or nothing (of 1,041), give or take tens of MiB that the runtime takes and returns by itself:
+    on which side of half the scratch it lies."""
+    import torch
+    from edgefem_amd import _capi
+    ring = 50
+    ang = 2 * np.pi * np.arange(ring) / ring
+    k, i = (v.ravel() for v in np.meshgrid(np.arange(levels), np.arange(ring), indexing="ij"))
+    xyz = np.concatenate([np.stack([np.zeros(levels + 1), np.zeros(levels + 1), np.arange(levels + 1.0)], 1),
+                          np.stack([np.cos(ang)[i], np.sin(ang)[i], k + 0.5], 1)])
+    base = levels + 1 + k * ring
+    tets = np.stack([k, k + 1, base + i, base + (i + 1) % ring], 1).astype(np.int32)
+    topo = _capi.Topology(np.arange(len(xyz)), tets, np.zeros((0, 3), np.int32))
+    scratch = len(tets) * 336
+    assert (scratch <= 2 ** 30) == keeps
+    xyz0, tets0 = _fan_mesh(3, 7)
+    small = _capi.Topology(np.arange(len(xyz0)), tets0, np.zeros((0, 3), np.int32))
+    _capi.assemble_km(small, xyz0, np.full(len(tets0), 2.0 + 0j))   # the runtime's first allocations
+    torch.cuda.synchronize()
+    held = lambda: -torch.cuda.mem_get_info()[0] - torch.cuda.memory_reserved()   # noqa: E731
+    before = held()
+    for _ in range(2):
+        K, M = _capi.assemble_km(topo, xyz, np.full(len(tets), 2.0 + 0j))
+    torch.cuda.synchronize()
+    got = held() - before
+    print(f"{len(tets)} tets: scratch {scratch / 2**20:.0f} MiB, held after {got / 2**20:.0f} MiB", flush=True)
+    assert (got > scratch / 2) == keeps
