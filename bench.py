@@ -724,7 +724,7 @@ def main():
     args = ap.parse_args()
     if args.traffic_from:
         cmd = ("rocprofv3 --pmc {c} --output-format csv -d pmc_{d} -o {d} -- python -u bench.py --no-cpu "
-               "--no-check --steps 1 --warmup 0 --max-it 20 --spmv-variant {v} --calibrate-copy 512")
+               "--no-check --no-extra --steps 1 --warmup 0 --max-it 20 --spmv-variant {v} --calibrate-copy 512")
         v = args.spmv_variant if args.spmv_variant >= 0 else 11
         traffic_from_pmc(args.traffic_from[0], args.traffic_from[1], os.path.join(ROOT, "profiles", "traffic_c2.json"),
                          v, [cmd.format(c="FETCH_SIZE", d="fetch", v=v), cmd.format(c="WRITE_SIZE", d="write", v=v)])
@@ -796,10 +796,13 @@ def main():
     s_val = 16 if args.mode == "fp64" else 8
     # algorithmic bytes of the chosen SpMV: the fused form reads z and p_old and writes p and
     # q per row and RHS (4 passes); variants 9-11 (p formed in its own pass, tiled, sliced-ELL
-    # or staged in LDS) gather p and write q (2 passes); the ELL padding slots are
-    # not algorithmic bytes, and variant 11's saving (8 B instead of 16 per real value) is
-    # not subtracted: the bytes are those of a complex value per entry
+    # or staged in LDS) gather p and write q (2 passes).  Padding slots are not algorithmic
+    # bytes.  Variant 11 reads 8 bytes per real part and 8 per imaginary part that is not zero;
+    # with staged columns an entry has a 2-byte index, and a row its place and its own index.
     spmv_bytes = nnz * (s_val + 4) + 4 * (n + 1) + R * n * 16 * (2 if variant in (9, 10, 11) else 4)
+    if variant == 11:
+        real = int((pipe.last_A.imag == 0).sum())
+        spmv_bytes -= 8 * real + (2 * nnz if staged else 0)
     avg_ms = spmv_ms / max(spmv_n, 1)
     achieved = spmv_bytes / (avg_ms * 1e-3)
     iters = int(max(pipe.last_info["iters"]))
