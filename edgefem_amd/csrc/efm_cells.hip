@@ -75,22 +75,24 @@ template <bool Y_OUTER> __device__ inline double norm2(double2 a) {
 }
 
 // block sum of V complex values over the first kBlock threads; result in lds[0..V) for all
-// threads (lds: V per wavefront of the block)
+// threads
 template <int V>
 __device__ inline void bsum(double2 (&v)[V], double2 *lds) {
-#pragma unroll
-  for (int s = 0; s < V; ++s) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-      v[s].x += __shfl_xor(v[s].x, off, 64);
-      v[s].y += __shfl_xor(v[s].y, off, 64);
-    }
-  }
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (lane == 0)
+  if (w < kBlock / 64) {
 #pragma unroll
-    for (int s = 0; s < V; ++s)
-      lds[w * V + s] = v[s];
+    for (int s = 0; s < V; ++s) {
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) {
+        v[s].x += __shfl_xor(v[s].x, off, 64);
+        v[s].y += __shfl_xor(v[s].y, off, 64);
+      }
+    }
+    if (lane == 0)
+#pragma unroll
+      for (int s = 0; s < V; ++s)
+        lds[w * V + s] = v[s];
+  }
   __syncthreads();
   if (threadIdx.x == 0)
 #pragma unroll
@@ -624,8 +626,10 @@ __global__ void __launch_bounds__(kBlock)
                 const double2 *__restrict__ out, const double2 *__restrict__ other, double2 *__restrict__ partial,
                 const CellSys *__restrict__ st) {
   constexpr int V = MODE == 0 ? R : 2 * R;
+  constexpr int U = 4;
   __shared__ double2 lo[R * kRowsPerTile], lt[R * kRowsPerTile];
   __shared__ double2 lds[(kBlock / 64) * 2 * kMaxR];
+  __shared__ int first[kRowsPerTile + 1];  // of every sub-tile, in the tile
   const Tile t = tiles[blockIdx.x];
   if (!cell_active<R>(st, t.cell))
     return;
@@ -641,6 +645,9 @@ __global__ void __launch_bounds__(kBlock)
     lo[i] = out[k];
     lt[i] = other[k];
   }
+  const int j0 = soff[blockIdx.x], nj = soff[blockIdx.x + 1] - j0;  // a sub-tile has a row: nj <= kRowsPerTile
+  for (int j = threadIdx.x; j <= nj; j += kBlock)
+    first[j] = j < nj ? (int)(sdesc[j0 + j].x - t.r0) : m / R;
   double2 d[V];
 #pragma unroll
   for (int s = 0; s < V; ++s)
@@ -648,23 +655,32 @@ __global__ void __launch_bounds__(kBlock)
   __syncthreads();
   const int g = threadIdx.x / kSubRL;
   if (threadIdx.x % kSubRL == 0)
-    for (int j = soff[blockIdx.x]; j < soff[blockIdx.x + 1]; ++j) {
-      const int4 dsc = sdesc[j];
-      if (dsc.x + g >= dsc.y)
-        continue;
-      const int i = (int)(dsc.x + g - t.r0) * R;
+    for (int j = 0; j < nj; j += U) {
+      double2 a[U][R], o[U][R];
+      bool in[U];
 #pragma unroll
-      for (int s = 0; s < R; ++s) {
-        if (!act[s])
-          continue;
-        const double2 a = lo[i + s], o = lt[i + s];
-        if (MODE == 0) {
-          d[s] = cfma(cconj(o), a, d[s]);
-        } else {
-          d[s] = cfma(cconj(a), o, d[s]);
-          d[R + s].x += norm2<R == 1>(a);
+      for (int u = 0; u < U; ++u) {
+        const int jj = min(j + u, nj - 1), r = first[jj] + g;
+        in[u] = j + u < nj && r < first[jj + 1];
+#pragma unroll
+        for (int s = 0; s < R; ++s) {
+          a[u][s] = lo[(in[u] ? r : 0) * R + s];
+          o[u][s] = lt[(in[u] ? r : 0) * R + s];
         }
       }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int s = 0; s < R; ++s) {
+          if (!in[u] || !act[s])
+            continue;
+          if (MODE == 0) {
+            d[s] = cfma(cconj(o[u][s]), a[u][s], d[s]);
+          } else {
+            d[s] = cfma(cconj(a[u][s]), o[u][s], d[s]);
+            d[R + s].x += norm2<R == 1>(a[u][s]);
+          }
+        }
     }
   put_partials<V>(d, lds, partial, blockIdx.x);
 }
@@ -774,7 +790,7 @@ __global__ void __launch_bounds__(NT)
               const double2 *__restrict__ tvec, const double2 *__restrict__ r0, double2 *__restrict__ x,
               double2 *__restrict__ r, double2 *__restrict__ partial, const CellSys *__restrict__ st) {
   constexpr bool kStaged = NT > kBlock;
-  __shared__ double2 lds[(NT / 64) * 2 * kMaxR];
+  __shared__ double2 lds[(kBlock / 64) * 2 * kMaxR];
   __shared__ double2 ldr[kStaged ? R * kRowsPerTile : 1];
   __shared__ double lrr[kStaged ? R * kRowsPerTile : 1];
   const Tile t = tiles[blockIdx.x];
