@@ -1684,14 +1684,26 @@ FlatDims flat_dims(int B) {
   return d;
 }
 
-// The packed kernels where the others would leave more than 3/8 of the lanes of one wavefront
-// or 1/4 of two or three idle (31 k rows, others against packed, ms: 6 systems 70, 30; 18: 61,
-// 41; 34: 63, 54; 40: 63, 61; 48: 65, 68; 66: 114, 83; 88: 111, 96; 96: 114, 110; 128: 123, 138;
-// 144: 176, 156; 4.8 k rows: 10 systems 17, 14; 40 and 80 17, 17 and 25, 24; 45 k rows: 40 and 96
-// systems 93, 92 and 181, 182), so for at most 143 systems; offsets in bytes in 32 bits.
+// The packed kernels where they are the faster ones: up to a number of systems in the last
+// wavefront that grows with the rows.  Small meshes are bound by latency, of which the packed
+// kernels have more (two barriers per chunk); on large ones the others pay for idle lanes.
+// Time per iteration, others over packed:
+//   rows     2 systems  18    32    36    38    76    88    95    136   143
+//   1.4 k    0.80       0.81  0.81  0.83        0.98              1.15
+//   4.3 k    1.03       0.98  0.97  0.90        0.92              0.99  0.97
+//   6.6 k    1.18       1.1   1.00  0.93  0.94  1.07  1.03  0.96  1.02  0.98
+//   13.7 k   1.66       1.3   1.09  1.01  0.93  1.12  1.08  0.92  1.05  1.02
+//   31 k     2.7        1.5   1.19  1.10  1.02  1.28  1.23  1.10  1.18  1.13
+//   46 k     3.7        1.7   1.24  1.11  1.06  1.24  1.18  0.98  1.19  1.13
+//   103 k    5.8        2.3   1.45  1.32  1.22  1.23  1.11  0.97        1.07
+// Offsets in bytes in 32 bits.
 bool flat_wins(int64_t n, int nsys) {
-  const int padded = (nsys + kSys - 1) / kSys * kSys;
-  return 8 * nsys < (padded > kSys ? 6 : 5) * padded && nsys <= 143 && n * nsys < ((int64_t)1 << 28);
+  constexpr int kMost[3][3] = {{32, 76, 136}, {36, 88, 143}, {38, 90, 143}};  // of one, two and three wavefronts
+  constexpr int64_t kRows[3] = {6000, 12000, 24000};
+  if (n < kRows[0] || nsys > 3 * kSys || n * nsys >= ((int64_t)1 << 28))
+    return false;
+  const int tier = n >= kRows[2] ? 2 : n >= kRows[1] ? 1 : 0;
+  return nsys <= kMost[tier][(nsys - 1) / kSys];
 }
 
 // Chunks of RB rows, contiguous per XCD (block bx runs on XCD bx % 8).

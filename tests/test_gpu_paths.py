@@ -391,15 +391,21 @@ def _fan_mesh(levels, ring):
 
 
 @pytest.mark.parametrize("graph", [False, True])
-@pytest.mark.parametrize("nsys,levels,ring,lossy", [
-    (1, 3, 7, False), (2, 40, 9, True), (18, 5, 60, False), (39, 4, 30, True), (65, 2, 30, False),
-    (95, 3, 20, False), (143, 2, 60, True)])
-def test_packed_sweep_batches(torch_dev, nsys, levels, ring, lossy, graph):
-    """Sweeps whose systems are packed into wavefronts: one system to three wavefronts of
-    them, chunks with more entries than are staged, real and complex matrices, two ports, a
+@pytest.mark.parametrize("nsys,levels,ring,lossy,packed", [
+    (1, 3, 7, False, False), (2, 40, 9, True, False), (18, 5, 60, False, False), (39, 4, 30, True, False),
+    (65, 2, 30, False, False), (95, 3, 20, False, False), (143, 2, 60, True, False),
+    (1, 34, 60, False, True), (2, 270, 9, True, True), (18, 34, 60, False, True), (32, 67, 30, True, True),
+    (33, 67, 30, True, False), (36, 134, 30, False, True), (37, 134, 30, False, False), (38, 134, 60, True, True),
+    (39, 134, 60, False, False), (65, 67, 30, False, True), (76, 34, 60, True, True), (77, 34, 60, True, False),
+    (88, 134, 30, False, True), (89, 134, 30, False, False), (90, 134, 60, False, True), (91, 134, 60, False, False),
+    (129, 34, 60, False, True), (136, 67, 30, True, True), (137, 67, 30, False, False), (143, 67, 60, True, True),
+    (144, 67, 60, False, False)])
+def test_packed_sweep_batches(torch_dev, nsys, levels, ring, lossy, packed, graph):
+    """Sweeps whose systems are packed into wavefronts, and those on the other side of the rule
+    (fewer rows, more systems): one system to three wavefronts of them, chunks with more entries than are staged, real and complex matrices, two ports, a
     right-hand side of zeros, eager and replayed.  tol = 1e-10; the recursive residual drifts
-    from the true one by iterations (below 200) times eps times the condition of the scaled
-    matrix (below 1e3): 2e-10 in all.  After 5 iterations the result agrees with the padded
+    from the true one by iterations (below 400 on the meshes of more than 6,000 rows) times eps
+    times the condition of the scaled matrix (below 1e3), 0.9e-10: 2e-10 in all.  After 5 iterations the result agrees with the padded
     kernels to the rounding of 5 sums of n terms times that condition, below 1e-9."""
     import torch
     import scipy.sparse as sp
@@ -429,7 +435,8 @@ def test_packed_sweep_batches(torch_dev, nsys, levels, ring, lossy, graph):
             X[pinned, cap] = X[pinned, cap].cpu().numpy().reshape(n, nsys)
             if cap == 10000:
                 iters = info["iters"]
-        assert sweep.variants()[:2] == ((1, 1) if pinned else (-1, -1))
+        got = sweep.variants()[:2]
+        assert got == (1, 1) if pinned else (got == (-1, -1)) == packed
     csr = lambda v: sp.csr_matrix((v, col, ptr), shape=(n, n))   # noqa: E731
     Y = X[False, 10000]
     r = B - csr(K.cpu().numpy()) @ Y + (csr(M.cpu().numpy()) @ Y) * k2
@@ -439,7 +446,7 @@ def test_packed_sweep_batches(torch_dev, nsys, levels, ring, lossy, graph):
     rel = (np.linalg.norm(r, axis=0)[on] / np.linalg.norm(B, axis=0)[on]).max()
     d = np.abs(X[False, 5] - X[True, 5]).max() / np.abs(X[True, 5]).max()
     print(f"n {n} nsys {nsys}: iterations {iters.max()} true {rel:.1e}; 5 iterations against padded {d:.1e}", flush=True)
-    assert iters.max() < 200 and rel <= 2e-10 and np.all(Y[:, ~on] == 0)
+    assert iters.max() < 400 and rel <= 2e-10 and np.all(Y[:, ~on] == 0)
     assert d <= 1e-9
 
 
@@ -449,7 +456,7 @@ def test_narrow_batch_after_a_wide_one(torch_dev, graph):
     same bits, and a wide one after it runs what was chosen; pinned variants stay pinned."""
     import torch
     from edgefem_amd import _capi
-    xyz, tets = _fan_mesh(6, 24)
+    xyz, tets = _fan_mesh(34, 60)
     topo = _capi.Topology(np.arange(len(xyz)), tets, np.zeros((0, 3), np.int32))
     n = topo.n_edges
     rng = np.random.default_rng(3)
