@@ -3079,8 +3079,8 @@ extern "C" int efm_solver_solve(efm_solver *s, const double *B, double *X,
   };
   if ((rc = start()) != EFM_OK)
     return rc;
-  // Systems whose matrix fits in the register files run in the persistent kernel: 780 rows 21.6
-  // (five launches) against 13.3 us per iteration, 31 k 29 against 18.4, 103 k 43 against 33.0.
+  // Systems whose matrix fits in the register files run in the persistent kernel: 780 rows 22.1
+  // (five launches) against 11.7 us per iteration, 31 k 27.5 against 18.0, 103 k 37.4 against 32.9.
   bool persist = false;
   if (cocg && !s->profile && (s->spmv_variant < 0 || s->tuned)) {
     rc = with_rhs(s->R, [&](auto RC) -> int {

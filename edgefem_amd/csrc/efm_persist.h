@@ -2,10 +2,12 @@
 //
 // On systems of up to about 10^5 rows every kernel of an iteration is a chain of a few
 // memory round trips behind a launch: 4-8 us each, five per iteration, whatever the size.
-// Here one launch runs all iterations.  Two right-hand sides, us per iteration, five launches
-// against this kernel: 780 rows 21.6, 13.3; 4.3 k 24, 14.1; 31 k 29, 18.4; 103 k 43, 33.0.  Of
-// the 18.4 us (123 blocks) the two grid sums take 6.8 and 5.7, the third barrier 3.2, the
-// nodal part 1.6 and the product 1.4: what is left is waiting, not work.
+// Here one launch runs all iterations.  us per iteration with two right-hand sides, the best
+// variant in launches against this kernel: 780 rows 22.1, 11.7; 4.3 k 23.5, 13.1; 31 k 27.5, 18.0;
+// 103 k 37.4, 32.9; 130 k 40.8, 37.7.  31 k rows, one right-hand side 20.7, 14.1; three 33.8, 26.3;
+// four 41.2, 36.1; two with two low-rank terms 35.1, 29.9 (103 k: 51.5, 49.6).  Of the 18 us (123
+// blocks) about two thirds are the two grid sums and a sixth the third barrier: what is left is
+// waiting, not work.
 // Block b owns rpb consecutive rows: their z, r, p live in registers of their element's
 // thread, their matrix entries in registers of their row's lanes (kRL lanes per row, kJ
 // entries each; longer rows read the rest from memory), so an iteration moves only what

@@ -402,11 +402,13 @@ def _fan_mesh(levels, ring):
     (144, 67, 60, False, False)])
 def test_packed_sweep_batches(torch_dev, nsys, levels, ring, lossy, packed, graph):
     """Sweeps whose systems are packed into wavefronts, and those on the other side of the rule
-    (fewer rows, more systems): one system to three wavefronts of them, chunks with more entries than are staged, real and complex matrices, two ports, a
-    right-hand side of zeros, eager and replayed.  tol = 1e-10; the recursive residual drifts
-    from the true one by iterations (below 400 on the meshes of more than 6,000 rows) times eps
-    times the condition of the scaled matrix (below 1e3), 0.9e-10: 2e-10 in all.  After 5 iterations the result agrees with the padded
-    kernels to the rounding of 5 sums of n terms times that condition, below 1e-9."""
+    (fewer rows, more systems): one system to three wavefronts of them, chunks with more
+    entries than are staged, real and complex matrices, two ports, a right-hand side of zeros,
+    eager and replayed.  tol = 1e-10; the recursive residual drifts from the true one by
+    iterations (below 400 on the meshes of more than 6,000 rows) times eps times the condition of
+    the scaled matrix (below 1e3), 0.9e-10: 2e-10 in all.  After 5 iterations the result agrees
+    with the padded kernels to the rounding of 5 sums of n terms times that condition, below
+    1e-9."""
     import torch
     import scipy.sparse as sp
     from edgefem_amd import _capi
