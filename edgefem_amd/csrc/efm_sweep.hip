@@ -1684,22 +1684,23 @@ FlatDims flat_dims(int B) {
   return d;
 }
 
-// The packed kernels where they are the faster ones: up to a number of systems in the last
-// wavefront that grows with the rows.  Small meshes are bound by latency, of which the packed
-// kernels have more (two barriers per chunk); on large ones the others pay for idle lanes.
-// Time per iteration, others over packed:
-//   rows     2 systems  18    32    36    38    76    88    95    136   143
-//   1.4 k    0.80       0.81  0.81  0.83        0.98              1.15
-//   4.3 k    1.03       0.98  0.97  0.90        0.92              0.99  0.97
-//   6.6 k    1.18       1.1   1.00  0.93  0.94  1.07  1.03  0.96  1.02  0.98
-//   13.7 k   1.66       1.3   1.09  1.01  0.93  1.12  1.08  0.92  1.05  1.02
-//   31 k     2.7        1.5   1.19  1.10  1.02  1.28  1.23  1.10  1.18  1.13
-//   46 k     3.7        1.7   1.24  1.11  1.06  1.24  1.18  0.98  1.19  1.13
-//   103 k    5.8        2.3   1.45  1.32  1.22  1.23  1.11  0.97        1.07
-// Offsets in bytes in 32 bits.
+// The packed kernels where they are the faster ones.  Small meshes are bound by latency, of which
+// the packed kernels have more (two barriers per chunk); on large ones the others pay for idle
+// lanes, and on all of them for the timing of their variants.  Time of a whole sweep on a new
+// object, others over packed:
+//   rows    10 systems  32    36    38    66    76    88    92    130   142
+//   1.6 k   0.93        0.99  0.95  0.95  1.02  1.04  1.03  1.02  1.05  1.03
+//   3.1 k   0.95        0.97  0.96  0.96  1.07  1.05  1.01  1.01  1.08  1.05
+//   5.1 k   1.07        1.04  1.01  1.04  1.07  1.05  1.05  1.05  1.10  1.05
+//   6.6 k   1.12        1.08  1.02  1.02  1.15  1.11  1.10  1.08  1.12  1.08
+//   8.1 k   1.21        1.08  1.00  0.97  1.13  1.09  1.04  1.03  1.12  1.08
+//   13 k    1.28        1.12  1.07  1.02  1.21  1.14  1.07  0.98  1.07  1.04
+//   44 k    2.09        1.26  1.22  1.08  1.52  1.28  1.15  0.98  1.17  1.06
+// (up to 0.03 of it set-up that has got faster since; 0.3 to 0.6 k rows: 0.67 to 0.77 with one
+// wavefront, 0.79 to 0.92 with more).  Offsets in bytes in 32 bits.
 bool flat_wins(int64_t n, int nsys) {
-  constexpr int kMost[3][3] = {{32, 76, 136}, {36, 88, 143}, {38, 90, 143}};  // of one, two and three wavefronts
-  constexpr int64_t kRows[3] = {6000, 12000, 24000};
+  constexpr int64_t kRows[3] = {3000, 6000, 12000};                               // at least
+  constexpr int kMost[3][3] = {{0, 95, 143}, {32, 95, 143}, {38, 88, 143}};  // of one, two and three wavefronts
   if (n < kRows[0] || nsys > 3 * kSys || n * nsys >= ((int64_t)1 << 28))
     return false;
   const int tier = n >= kRows[2] ? 2 : n >= kRows[1] ? 1 : 0;

@@ -306,9 +306,9 @@ int efm_sweep_solve(efm_sweep *sw, int nsys, const double *h_k0sq, const double 
  * LDS-tiled: each tile of 8 consecutive rows loads its distinct columns (at most 72)
  * once per group of 64 systems into LDS and its rows read them there; available when
  * every tile fits (set returns an error otherwise); -1 (default) = with form 2, no
- * reliable updates, at least 6,000 rows and a batch that would leave many of its wavefronts'
- * lanes idle (up to 32, 65-76 and 129-136 systems; from 12,000 rows 36, 88 and 143; from
- * 24,000 rows 38, 90 and 143), kernels that pack the systems of several rows into a
+ * reliable updates, at least 3,000 rows and a batch that would leave many of its wavefronts'
+ * lanes idle (65-95 and 129-143 systems; from 6,000 rows also up to 32; from 12,000 rows up
+ * to 38, 65-88 and 129-143), kernels that pack the systems of several rows into a
  * wavefront (get reports -1); otherwise the fastest, chosen on the first such solve: the
  * iterations before its first convergence check cycle through the candidates, each launch
  * timed in place.  The choice does not change which batches are packed.  get: the variants

@@ -394,12 +394,12 @@ def _fan_mesh(levels, ring):
 @pytest.mark.parametrize("nsys,levels,ring,lossy,packed", [
     (1, 3, 7, False, False), (2, 40, 9, True, False), (18, 5, 60, False, False), (39, 4, 30, True, False),
     (65, 2, 30, False, False), (95, 3, 20, False, False), (143, 2, 60, True, False),
+    (32, 33, 30, False, False), (65, 32, 30, False, False), (65, 33, 30, False, True), (95, 33, 30, True, True),
+    (96, 33, 30, False, False), (143, 33, 30, True, True), (144, 33, 30, False, False),
     (1, 34, 60, False, True), (2, 270, 9, True, True), (18, 34, 60, False, True), (32, 67, 30, True, True),
-    (33, 67, 30, True, False), (36, 134, 30, False, True), (37, 134, 30, False, False), (38, 134, 60, True, True),
-    (39, 134, 60, False, False), (65, 67, 30, False, True), (76, 34, 60, True, True), (77, 34, 60, True, False),
-    (88, 134, 30, False, True), (89, 134, 30, False, False), (90, 134, 60, False, True), (91, 134, 60, False, False),
-    (129, 34, 60, False, True), (136, 67, 30, True, True), (137, 67, 30, False, False), (143, 67, 60, True, True),
-    (144, 67, 60, False, False)])
+    (33, 67, 30, True, False), (95, 34, 60, True, True), (129, 34, 60, False, True), (136, 67, 30, True, True),
+    (38, 134, 30, False, True), (39, 134, 30, False, False), (88, 134, 30, True, True), (89, 134, 30, False, False),
+    (143, 67, 60, True, True), (144, 67, 60, False, False)])
 def test_packed_sweep_batches(torch_dev, nsys, levels, ring, lossy, packed, graph):
     """Sweeps whose systems are packed into wavefronts, and those on the other side of the rule
     (fewer rows, more systems): one system to three wavefronts of them, chunks with more
